@@ -78,7 +78,12 @@ inline void launch_k(int prof_id, void (*kern)(P...), dim3 grid, dim3 block, siz
 }
 
 // bookkeeping of isos_update (sealevel.f90, fastisostasy.f90:750-833)
-void launch_pre_haf(const Member* d_mem, int nmem, int n, bool new_H, hipStream_t st);
+// ice: the new ice thickness of a single domain in pinned host memory, or null
+// (every member's H_in holds its ice)
+void launch_pre_haf(const Member* d_mem, int nmem, int n, const double* ice, hipStream_t st);
+// rows [j0, j0 + nj) x columns [i0, i0 + ni) of an n x n field into dst (contiguous
+// doubles), or, with bit != 0, of that bit of an n x n byte mask (contiguous bytes 0 / 1)
+void launch_crop(const void* src, int bit, int n, int i0, int j0, int ni, int nj, void* dst, hipStream_t st);
 void launch_pre_bsl(const Member* d_mem, int nmem, int n, hipStream_t st);
 // phase 0: z_ss/masks/loads and, without diagnostics, everything the RHS needs
 // phase 1: (after the elastic convolution) litho/full/mass anomaly

@@ -51,7 +51,11 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
     return s;
 }
 
-__global__ void __launch_bounds__(PRE_THREADS) k_pre_haf(const Member* __restrict__ mem, int new_H) {
+// ice: one domain's new ice thickness, read over the bus from pinned host
+// memory (256^2: 0.5 MB); H_in then receives it for later updates without new
+// ice.  Null: H_in holds the ice already.
+template <bool HOST>
+__global__ void __launch_bounds__(PRE_THREADS) k_pre_haf(const Member* __restrict__ mem, const double* __restrict__ ice) {
     const Member& M = mem[blockIdx.y];
     const kptr<PhysDev> ph = kview(M.phys);
     const int N = M.n;
@@ -59,28 +63,31 @@ __global__ void __launch_bounds__(PRE_THREADS) k_pre_haf(const Member* __restric
     double s1 = 0.0, s2 = 0.0;
     const double A_uni = ph->dx * ph->dx, Vden = ph->Vden_factor, rsw_ri = ph->rho_seawater / ph->rho_ice;
     const bool uniform = ph->uniform_K;
-    gptr<double> Hin = gin<double>(M.H_in), zss = gin<double>(M.z_ss), zbed = gin<double>(M.z_bed),
+    gptr<double> Hin = gin<double>(HOST ? ice : M.H_in), zss = gin<double>(M.z_ss), zbed = gin<double>(M.z_bed),
                  Haf_ref = gin<double>(M.Haf_ref), Hice_ref = gin<double>(M.Hice_ref);
-    gmut<double> Hice = gout<double>(M.Hice), Haf = gout<double>(M.Haf);
+    gmut<double> Hice = gout<double>(M.Hice), Haf = gout<double>(M.Haf), Hkeep = gout<double>(M.H_in);
     // every load of the thread's cells first (indices clamped, so no branch),
     // then the arithmetic and the guarded stores
     constexpr int IT = PRE_CELLS / PRE_THREADS;
     double Hv[IT], zs[IT], zb[IT], hr[IT], ir[IT], Av[IT];
     bool inside[IT];
+    size_t at[IT];
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-        size_t c = (size_t)blockIdx.x * PRE_CELLS + it * PRE_THREADS + threadIdx.x;
-        c = c < nn ? c : nn - 1;
-        if (new_H) {
-            // out2in embedding of the ice grid (isos_utils.f90:330-345)
-            const int i = (int)(c % N) - M.icrop1, j = (int)(c / N) - M.jcrop1;
-            inside[it] = i >= 0 && i < M.nx_ice && j >= 0 && j < M.ny_ice;
-            const int ic = i < 0 ? 0 : (i >= M.nx_ice ? M.nx_ice - 1 : i);
-            const int jc = j < 0 ? 0 : (j >= M.ny_ice ? M.ny_ice - 1 : j);
-            Hv[it] = Hin[(size_t)jc * M.nx_ice + ic];
+        const size_t cr = (size_t)blockIdx.x * PRE_CELLS + it * PRE_THREADS + threadIdx.x;
+        const size_t c = cr < nn ? cr : nn - 1;
+        // out2in embedding of the ice grid (isos_utils.f90:330-345)
+        const int i = (int)(c % N) - M.icrop1, j = (int)(c / N) - M.jcrop1;
+        inside[it] = i >= 0 && i < M.nx_ice && j >= 0 && j < M.ny_ice;
+        const int ic = i < 0 ? 0 : (i >= M.nx_ice ? M.nx_ice - 1 : i);
+        const int jc = j < 0 ? 0 : (j >= M.ny_ice ? M.ny_ice - 1 : j);
+        at[it] = (size_t)jc * M.nx_ice + ic;
+        // (cells of the padding read nothing over the bus)
+        if constexpr (HOST) {
+            Hv[it] = 0.0;
+            if (inside[it] && cr < nn) Hv[it] = Hin[at[it]];
         } else {
-            inside[it] = true;
-            Hv[it] = Hice[c];
+            Hv[it] = Hin[at[it]];
         }
         zs[it] = zss[c]; zb[it] = zbed[c]; hr[it] = Haf_ref[c]; ir[it] = Hice_ref[c];
         Av[it] = uniform ? A_uni : M.A[c];
@@ -90,7 +97,9 @@ __global__ void __launch_bounds__(PRE_THREADS) k_pre_haf(const Member* __restric
         const size_t c = (size_t)blockIdx.x * PRE_CELLS + it * PRE_THREADS + threadIdx.x;
         if (c >= nn) break;
         const double H = inside[it] ? Hv[it] : 0.0;
-        if (new_H) Hice[c] = H;
+        Hice[c] = H;
+        if constexpr (HOST)
+            if (inside[it]) Hkeep[at[it]] = H;
         // calc_Haf (sealevel.f90:132-145)
         double h = (zs[it] - zb[it]) * rsw_ri;
         if (h < 0.0) h = 0.0;
@@ -488,8 +497,34 @@ __global__ void __launch_bounds__(PRE_THREADS) k_init_state(const Member* __rest
 // ------------------------------------------------------------------ launchers
 static int pre_blocks(int n) { return (int)(((size_t)n * n + PRE_CELLS - 1) / PRE_CELLS); }
 
-void launch_pre_haf(const Member* d_mem, int nmem, int n, bool new_H, hipStream_t st) {
-    hipLaunchKernelGGL(k_pre_haf, dim3(pre_blocks(n), nmem), dim3(PRE_THREADS), 0, st, d_mem, (int)new_H);
+void launch_pre_haf(const Member* d_mem, int nmem, int n, const double* ice, hipStream_t st) {
+    const dim3 g(pre_blocks(n), nmem), b(PRE_THREADS);
+    if (ice) hipLaunchKernelGGL(k_pre_haf<true>, g, b, 0, st, d_mem, ice);
+    else hipLaunchKernelGGL(k_pre_haf<false>, g, b, 0, st, d_mem, ice);
+}
+
+// Window of a field (or of one mask bit) packed row by row, for pinned host
+// memory: consecutive lanes store consecutive values, so a wave's store is one
+// run of 512 (64) bytes on the bus.
+__global__ void __launch_bounds__(256) k_crop(const double* __restrict__ src, int n, int i0, int j0, int ni, int count,
+                                              double* __restrict__ dst) {
+    const int q = blockIdx.x * 256 + threadIdx.x;
+    if (q >= count) return;
+    dst[q] = src[(size_t)(j0 + q / ni) * n + i0 + q % ni];
+}
+__global__ void __launch_bounds__(256) k_crop_mask(const uint8_t* __restrict__ src, int bit, int n, int i0, int j0,
+                                                   int ni, int count, uint8_t* __restrict__ dst) {
+    const int q = blockIdx.x * 256 + threadIdx.x;
+    if (q >= count) return;
+    dst[q] = (src[(size_t)(j0 + q / ni) * n + i0 + q % ni] & bit) ? 1 : 0;
+}
+void launch_crop(const void* src, int bit, int n, int i0, int j0, int ni, int nj, void* dst, hipStream_t st) {
+    const int count = ni * nj;
+    const dim3 g((count + 255) / 256), b(256);
+    if (bit)
+        hipLaunchKernelGGL(k_crop_mask, g, b, 0, st, (const uint8_t*)src, bit, n, i0, j0, ni, count, (uint8_t*)dst);
+    else
+        hipLaunchKernelGGL(k_crop, g, b, 0, st, (const double*)src, n, i0, j0, ni, count, (double*)dst);
 }
 void launch_pre_bsl(const Member* d_mem, int nmem, int n, hipStream_t st) {
     hipLaunchKernelGGL(k_pre_bsl, dim3(nmem), dim3(64), 0, st, d_mem, nmem, pre_blocks(n));
