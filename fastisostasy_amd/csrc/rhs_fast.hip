@@ -621,32 +621,28 @@ __device__ __forceinline__ void row_reduce_store(double a1a, double a2a, double 
     constexpr int G = P2 ? TPL : TPL / 3;                  // lanes reduced by shuffles
     static_assert(P2 || (G * 3 == TPL && (G & (G - 1)) == 0 && G <= 64), "TPL = 2^j or 3 * 2^j");
     constexpr int W = G < 64 ? G : 64;
-#pragma unroll
-    for (int o = W / 2; o > 0; o >>= 1) {
-        a1a = fmax(a1a, __shfl_xor(a1a, o, W)); a2a = fmax(a2a, __shfl_xor(a2a, o, W));
-        s2a += __shfl_xor(s2a, o, W);
-        a1b = fmax(a1b, __shfl_xor(a1b, o, W)); a2b = fmax(a2b, __shfl_xor(a2b, o, W));
-        s2b += __shfl_xor(s2b, o, W);
-    }
+    // (only the largest of the four maxima is used: one butterfly for them)
+    a1a = lanes_max<W>(fmax(fmax(a1a, a2a), fmax(a1b, a2b)));
+    s2a = lanes_sum<W>(s2a);
+    s2b = lanes_sum<W>(s2b);
     constexpr int NG = P2 ? (TPL > 64 ? TPL / 64 : 1) : 3;   // groups combined through LDS
     if constexpr (NG > 1) {
-        __shared__ double red[16][NG][6];
+        __shared__ double red[16][NG][3];
         if ((t % W) == 0) {
             double* r = red[line][t / W];
-            r[0] = a1a; r[1] = a2a; r[2] = s2a; r[3] = a1b; r[4] = a2b; r[5] = s2b;
+            r[0] = a1a; r[1] = s2a; r[2] = s2b;
         }
         __syncthreads();
         if (t == 0) {
             for (int w = 1; w < NG; ++w) {
                 const double* r = red[line][w];
-                a1a = fmax(a1a, r[0]); a2a = fmax(a2a, r[1]); s2a += r[2];
-                a1b = fmax(a1b, r[3]); a2b = fmax(a2b, r[4]); s2b += r[5];
+                a1a = fmax(a1a, r[0]); s2a += r[1]; s2b += r[2];
             }
         }
     }
     if (t == 0) {
         // one entry per line: rows 2j and 2j+1 combined in a fixed order
-        pa[0] = fmax(fmax(a1a, a2a), fmax(a1b, a2b));
+        pa[0] = a1a;
         pa[1] = s2a + s2b;
     }
 }
