@@ -202,10 +202,9 @@ bool tuned_for(int n, bool fp64, int nmem, TunedShape& out) {
     return true;
 }
 
-// Row / column blocking for a batch of `nmem` domains of size n.
-int make_shape(int n, int nmem, bool fp64, bool uniform, RhsShape& s) {
-    TunedShape ts;
-    const bool tuned = tuned_for(n, fp64, nmem, ts);
+// Row / column blocking of the three-pass kernels (and of the mixed-radix LDS
+// kernels) for a batch of `nmem` domains of size n.
+int make_three_pass_shape(int n, int nmem, bool fp64, bool uniform, bool tuned, const TunedShape& ts, RhsShape& s) {
     if (!make_plan(n, s.plan))
         return fail(FI_E_UNSUPPORTED, "padded size N=%d has a prime factor > 7; choose pad so that N is 2^a 3^b 5^c 7^d", n);
     s.n = n;
@@ -382,6 +381,50 @@ int make_shape(int n, int nmem, bool fp64, bool uniform, RhsShape& s) {
     s.tw = fp64 ? (const void*)t.d64 : (const void*)t.d32;
     s.tw64 = t.d64;
     return 0;
+}
+
+// Two-launch attempts (rhs_turn.hpp) for this group?  At the general lengths
+// always: they replace five launches of the mixed-radix LDS kernels (one
+// N = 320 domain, mixed: 17.1 us per attempt against 59.5; 64 of 200^2: 62.5
+// against 155).  At the lengths of the three-launch register kernels (2^k,
+// 3 * 2^k) only for small groups that those serve with five launches: distorted
+// grids and N = 192 (uniform N = 192: 17.5 us against 26.9; uniform N = 256 is
+// a tie, 16.9 against 17.1).  A launch shape asked of the other kernels
+// (environment, autotuner) keeps those; FI_TURN = 0 never, 2 wherever the
+// kernels exist (tests).
+//
+// Blocks: one line pair per kt_turn block while two would leave CUs idle (N =
+// 320: 17.1 us against 18.7; 30 of 200^2: 39 against 49 the other way round),
+// 2 line pairs per kt_col block until 8 give every CU a block (30 of 200^2:
+// 39.4 us per attempt against 45.1).
+constexpr long long TURN_SMALL = 512;   // blocks of two line pairs
+
+void turn_shape(int n, int nmem, bool fp64, bool uniform, bool tuned, const TunedShape& ts, RhsShape& s) {
+    s.turn = nullptr;
+    s.turn_C = s.turn_LO = 2;
+    for (const char* e : {"FI_GENERIC_FFT", "FI_GEN_LINES", "FI_NO_FUSED_STENCIL", "FI_SROW_ROWS", "FI_INV_THREADS",
+                          "FI_ROW_THREADS", "FI_COL_LINES", "FI_ROW_TILES"})
+        if (std::getenv(e)) return;
+    const char* env = std::getenv("FI_TURN");
+    const int want = env ? std::atoi(env) : 1;
+    if (want == 0) return;
+    if (tuned && (ts.threads_row || ts.C || ts.row_tiles || ts.gL || ts.gC || ts.srow_rows || ts.threads_inv)) return;
+    const long long blocks = (long long)(n / 4) * nmem;
+    if (s.fast && want != 2 && ((uniform && n != 192) || blocks > TURN_SMALL)) return;
+    s.turn_C = blocks >= 1024 ? 8 : 2;
+    s.turn_LO = blocks >= 256 ? 2 : 1;
+    TurnFn f = turn_find(n, fp64);
+    // (a device that refuses the kernels' LDS keeps the others)
+    if (f && f(nullptr, nmem, s, nullptr, -1)) s.turn = f;
+}
+
+// Row / column blocking for a batch of `nmem` domains of size n.
+int make_shape(int n, int nmem, bool fp64, bool uniform, RhsShape& s) {
+    TunedShape ts;
+    const bool tuned = tuned_for(n, fp64, nmem, ts);
+    int rc = make_three_pass_shape(n, nmem, fp64, uniform, tuned, ts, s);
+    if (!rc) turn_shape(n, nmem, fp64, uniform, tuned, ts, s);
+    return rc;
 }
 
 int make_conv_shape(int n, bool fp64, ConvShape& s) {
@@ -720,7 +763,8 @@ bool same_shape(const RhsShape& a, const RhsShape& b) {
            a.threads_col == b.threads_col && a.fp64 == b.fp64 && a.uniform == b.uniform && a.fast == b.fast &&
            a.fused == b.fused && a.row_tiles == b.row_tiles && a.srow_rows == b.srow_rows &&
            a.threads_inv == b.threads_inv && a.tw == b.tw && a.tw64 == b.tw64 &&
-           a.plan.n == b.plan.n && a.plan.nf == b.plan.nf && a.method == b.method && a.dt_method == b.dt_method;
+           a.plan.n == b.plan.n && a.plan.nf == b.plan.nf && a.method == b.method && a.dt_method == b.dt_method && a.turn == b.turn &&
+           a.turn_C == b.turn_C && a.turn_LO == b.turn_LO;
 }
 
 int attempt_graph(const Member* d, int nmem, const RhsShape& s, hipStream_t st, hipGraphExec_t* out) {
@@ -899,12 +943,15 @@ int job_round(UpdateJob& j) {
     Member* d_mem = j.d_mem;
     if (j.stepping) {
         if (j.K == 1) {
+            launch_round_start(d_mem, nmem, shape, j.st);
             int rc = launch_attempts(d_mem, nmem, shape, j.st, j.ahead, j.graphs);
             if (rc) return rc;
             launch_decide(d_mem, nmem, shape, j.st);
         } else {
             HIPCHK(hipEventRecord(g_sub.start, j.st));
             for (int k = 0; k < j.K; ++k) HIPCHK(hipStreamWaitEvent(g_sub.s[k], g_sub.start, 0));
+            for (int k = 0; k < j.K; ++k)
+                launch_round_start(d_mem + j.sb_lo[k], j.sb_lo[k + 1] - j.sb_lo[k], *j.sshape[k], g_sub.s[k]);
             // interleave the sub-batches' launches so both queues fill together
             for (int a = 0; a < j.ahead; a += GRAPH_REPS)
                 for (int k = 0; k < j.K; ++k) {

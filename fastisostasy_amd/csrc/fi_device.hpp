@@ -15,6 +15,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "fi_types.h"
 
 namespace fi {
@@ -42,6 +44,14 @@ __device__ __forceinline__ cplx<float> cmul(cplx<float> a, cplx<float> b) {
 template <typename C> __device__ __forceinline__ C cmi(C a) { C r; r.x = a.y; r.y = -a.x; return r; }
 // multiply by +i
 template <typename C> __device__ __forceinline__ C cpi(C a) { C r; r.x = -a.y; r.y = a.x; return r; }
+
+// f(integral_constant<int, B>) ... f(integral_constant<int, E - 1>)
+template <int B, int E, class F> __device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (B < E) {
+        f(std::integral_constant<int, B>{});
+        static_for<B + 1, E>(f);
+    }
+}
 
 // ---------------------------------------------------------------- butterflies
 template <typename C> __device__ __forceinline__ void bfly2(C* v) {

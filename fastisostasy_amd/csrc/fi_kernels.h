@@ -10,6 +10,13 @@
 
 namespace fi {
 
+struct RhsShape;
+// Launches of the two-launch attempt of one length and precision (rhs_turn.hpp):
+// which = 0 forward part of a round's first attempt, 1 column pass, 2 turn;
+// -1 launches nothing and says whether the kernels can run on this device
+using TurnFn = bool (*)(const Member*, int, const RhsShape&, hipStream_t, int);
+TurnFn turn_find(int n, bool fp64);   // null: no such length
+
 // Launch geometry of one attempted step for a batch of equal-size domains.
 struct RhsShape {
     int n;
@@ -29,6 +36,9 @@ struct RhsShape {
     int threads_inv;  // fast: block size of the inverse row pass (0: threads_row)
     int method;       // 3 LV-ELVA (transform passes); 0-2 pointwise relaxation RHS
     int dt_method;    // integrator shared by the batch (0-3), -1 if not known
+    TurnFn turn;      // not null: attempts run as kt_col, kt_turn (rhs_turn.hpp)
+    int turn_C;       // line pairs per kt_col block (2 or 8)
+    int turn_LO;      // line pairs per kt_turn block (1 or 2)
 };
 
 // Geometry of the 2N-point linear convolution.
@@ -42,6 +52,8 @@ struct ConvShape {
     bool rows_twl;    // the row passes also hold the twiddle table in LDS (the column pass always does)
 };
 
+// before the first attempt of a launch round (two-launch attempts only)
+void launch_round_start(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st);
 void launch_attempt(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st);
 // applies a pending step decision left by the last attempt (no-op otherwise)
 void launch_decide(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st);

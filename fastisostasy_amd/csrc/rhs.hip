@@ -506,6 +506,27 @@ void launch_attempt_xlra(const Member* d_mem, int nmem, const RhsShape& s, hipSt
     hipLaunchKernelGGL(k_decide, dim3(nmem), dim3(64), 0, st, d_mem, nblk);
 }
 
+// two-launch attempts: lengths by translation unit
+TurnFn turn_part0(int, bool);
+TurnFn turn_part1(int, bool);
+TurnFn turn_part2(int, bool);
+TurnFn turn_part3(int, bool);
+TurnFn turn_part4(int, bool);
+TurnFn turn_part5(int, bool);
+TurnFn turn_part6(int, bool);
+TurnFn turn_part7(int, bool);
+TurnFn turn_find(int n, bool fp64) {
+    using Part = TurnFn (*)(int, bool);
+    constexpr Part parts[] = {turn_part0, turn_part1, turn_part2, turn_part3,
+                              turn_part4, turn_part5, turn_part6, turn_part7};
+    for (Part p : parts)
+        if (TurnFn f = p(n, fp64)) return f;
+    return nullptr;
+}
+void launch_round_start(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st) {
+    if (s.method == 3 && s.turn) s.turn(d_mem, nmem, s, st, 0);
+}
+
 template <typename T>
 void launch_attempt_t(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st) {
     dim3 gs((s.n + ST_TX - 1) / ST_TX, (s.n + ST_TY - 1) / ST_TY, nmem);
@@ -537,13 +558,19 @@ void launch_attempt_t(const Member* d_mem, int nmem, const RhsShape& s, hipStrea
 }
 
 void launch_decide(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st) {
-    // partials: one per line pair of rows on the power-of-two path, one per row otherwise
+    // partials: one per line pair of rows on the register kernels, one per row on the mixed-radix LDS kernels
     const int nblk = s.fast ? s.n / 2 : s.n;
     hipLaunchKernelGGL(k_decide, dim3(nmem), dim3(64), 0, st, d_mem, nblk);
 }
 
 void launch_attempt(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st) {
     if (s.method != 3) launch_attempt_xlra(d_mem, nmem, s, st);
+    else if (s.turn) {
+        g_prof.fused.store(true, std::memory_order_relaxed);
+        if (g_prof.kernel >= 0) g_prof.last = s;
+        s.turn(d_mem, nmem, s, st, 1);
+        s.turn(d_mem, nmem, s, st, 2);
+    }
     else if (s.fp64) launch_attempt_t<double>(d_mem, nmem, s, st);
     else launch_attempt_t<float>(d_mem, nmem, s, st);
 }

@@ -65,10 +65,12 @@ __device__ __forceinline__ double stage_sums_m(double x, double k, double dt, do
         return x + dt * (((0.0 * k + 0.0 * k) + 0.0 * k) + 3 * k);
     }
     // tsit54: b = (0.0845, 0, 0, 0.5179, 0.1276, 0.27), bh(6) = 0.27 - 1/5
+    // (the two terms of weight 0 change no sum; an infinite k still leaves a
+    // NaN in the error norm, from x2 - x1)
     const double b1 = dt * 0.0845, b4 = dt * 0.5179, b5 = dt * 0.1276, b6 = dt * 0.2700;
-    const double z = dt * 0.0, h6 = dt * (0.2700 - 1 / 5.0);
-    x1 = x + b1 * k + z * k + z * k + b4 * k + b5 * k + h6 * k;
-    return x + b1 * k + z * k + z * k + b4 * k + b5 * k + b6 * k;
+    const double h6 = dt * (0.2700 - 1 / 5.0);
+    x1 = x + b1 * k + b4 * k + b5 * k + h6 * k;
+    return x + b1 * k + b4 * k + b5 * k + b6 * k;
 }
 
 // the integrator as a run-time value
@@ -197,6 +199,59 @@ __device__ __forceinline__ void store_state(Ctl* c, const StepState& s) {
     c->t = s.t; c->dt = s.dt; c->tf = s.tf; c->err = s.err; c->tol = s.tol;
     c->cur = s.cur; c->w_is_x = s.w_is_x; c->k_valid = s.k_valid; c->status = s.status;
     c->attempts = s.attempts; c->accepts = s.accepts;
+}
+
+template <typename T> struct vec2;
+template <> struct vec2<float> { typedef float type __attribute__((ext_vector_type(2))); };
+template <> struct vec2<double> { typedef double type __attribute__((ext_vector_type(2))); };
+
+// (member, block-within-member) for a grid (blocks per member, members)
+__device__ __forceinline__ void xcd_order(int& member, int& blk) {
+    const int per = gridDim.x, total = gridDim.x * gridDim.y;
+    int b = blockIdx.x + per * blockIdx.y;
+    if ((total & 7) == 0) b = (b & 7) * (total >> 3) + (b >> 3);
+    member = b / per;
+    blk = b % per;
+}
+
+// Reduce the per-thread row statistics of two rows over the TPL threads of a
+// line with a fixed butterfly (lines wider than a wave combine their wave
+// halves through LDS in wave order; lines of 3 * 2^j threads combine their
+// three 2^j-lane groups through LDS in group order), and store them as the
+// row's partials.  The pattern depends on N alone, so the error norm of a
+// domain does not depend on how many domains share the launch.
+template <int TPL>
+__device__ __forceinline__ void row_reduce_store(double a1a, double a2a, double s2a, double a1b, double a2b,
+                                                 double s2b, int line, int t, gmut<double> pa,
+                                                 bool store = true) {
+    constexpr bool P2 = (TPL & (TPL - 1)) == 0;
+    constexpr int G = P2 ? TPL : TPL / 3;                  // lanes reduced by shuffles
+    static_assert(P2 || (G * 3 == TPL && (G & (G - 1)) == 0 && G <= 64), "TPL = 2^j or 3 * 2^j");
+    constexpr int W = G < 64 ? G : 64;
+    // (only the largest of the four maxima is used: one butterfly for them)
+    a1a = lanes_max<W>(fmax(fmax(a1a, a2a), fmax(a1b, a2b)));
+    s2a = lanes_sum<W>(s2a);
+    s2b = lanes_sum<W>(s2b);
+    constexpr int NG = P2 ? (TPL > 64 ? TPL / 64 : 1) : 3;   // groups combined through LDS
+    if constexpr (NG > 1) {
+        __shared__ double red[16][NG][3];
+        if ((t % W) == 0) {
+            double* r = red[line][t / W];
+            r[0] = a1a; r[1] = s2a; r[2] = s2b;
+        }
+        __syncthreads();
+        if (t == 0) {
+            for (int w = 1; w < NG; ++w) {
+                const double* r = red[line][w];
+                a1a = fmax(a1a, r[0]); s2a += r[1]; s2b += r[2];
+            }
+        }
+    }
+    if (t == 0 && store) {
+        // one entry per line: rows 2j and 2j+1 combined in a fixed order
+        pa[0] = a1a;
+        pa[1] = s2a + s2b;
+    }
 }
 
 // Stand-alone decision of one domain (one wave): applies the pending

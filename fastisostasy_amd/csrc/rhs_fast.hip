@@ -31,10 +31,6 @@ __device__ __forceinline__ void load_tw(cplx<T>* tw_l, const cplx<T>* __restrict
     for (int q = threadIdx.x; q < 2 * N; q += blockDim.x) l[q] = g[q];
 }
 
-template <typename T> struct vec2;
-template <> struct vec2<float> { typedef float type __attribute__((ext_vector_type(2))); };
-template <> struct vec2<double> { typedef double type __attribute__((ext_vector_type(2))); };
-
 template <typename T, int N, int THREADS>
 __global__ void __launch_bounds__(THREADS) kf_row_fwd(const Member* __restrict__ mem, const void* __restrict__ twv) {
     const Member& M = mem[blockIdx.y];
@@ -102,22 +98,6 @@ template <typename T, int N, int THREADS, int LF = THREADS / (N / 8)> struct SRo
 // (4: measured 23.7 us per launch on the 64-member ensemble against 24.9 at 6
 // and 25.7 at 8; nearer loads hold fewer registers)
 constexpr int SR_LA = 4;
-
-template <int B, int E, class F> __device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (B < E) {
-        f(std::integral_constant<int, B>{});
-        static_for<B + 1, E>(f);
-    }
-}
-
-// (member, block-within-member) for a grid (blocks per member, members)
-__device__ __forceinline__ void xcd_order(int& member, int& blk) {
-    const int per = gridDim.x, total = gridDim.x * gridDim.y;
-    int b = blockIdx.x + per * blockIdx.y;
-    if ((total & 7) == 0) b = (b & 7) * (total >> 3) + (b >> 3);
-    member = b / per;
-    blk = b % per;
-}
 
 // The march and the row transform of one block.  issue(tau) issues the
 // global loads due at march step tau (inputs arrive SR_LA steps ahead of use).
@@ -606,45 +586,6 @@ __global__ void __launch_bounds__(C * (N / 8)) kf_col(const Member* __restrict__
         }
     }
     if (commit) copy_ctl(M.ctl, c);
-}
-
-// Reduce the per-thread row statistics of two rows over the TPL threads of a
-// line with a fixed butterfly (lines wider than a wave combine their wave
-// halves through LDS in wave order; lines of 3 * 2^j threads combine their
-// three 2^j-lane groups through LDS in group order), and store them as the
-// row's partials.  The pattern depends on N alone, so the error norm of a
-// domain does not depend on how many domains share the launch.
-template <int TPL>
-__device__ __forceinline__ void row_reduce_store(double a1a, double a2a, double s2a, double a1b, double a2b,
-                                                 double s2b, int line, int t, gmut<double> pa) {
-    constexpr bool P2 = (TPL & (TPL - 1)) == 0;
-    constexpr int G = P2 ? TPL : TPL / 3;                  // lanes reduced by shuffles
-    static_assert(P2 || (G * 3 == TPL && (G & (G - 1)) == 0 && G <= 64), "TPL = 2^j or 3 * 2^j");
-    constexpr int W = G < 64 ? G : 64;
-    // (only the largest of the four maxima is used: one butterfly for them)
-    a1a = lanes_max<W>(fmax(fmax(a1a, a2a), fmax(a1b, a2b)));
-    s2a = lanes_sum<W>(s2a);
-    s2b = lanes_sum<W>(s2b);
-    constexpr int NG = P2 ? (TPL > 64 ? TPL / 64 : 1) : 3;   // groups combined through LDS
-    if constexpr (NG > 1) {
-        __shared__ double red[16][NG][3];
-        if ((t % W) == 0) {
-            double* r = red[line][t / W];
-            r[0] = a1a; r[1] = s2a; r[2] = s2b;
-        }
-        __syncthreads();
-        if (t == 0) {
-            for (int w = 1; w < NG; ++w) {
-                const double* r = red[line][w];
-                a1a = fmax(a1a, r[0]); s2a += r[1]; s2b += r[2];
-            }
-        }
-    }
-    if (t == 0) {
-        // one entry per line: rows 2j and 2j+1 combined in a fixed order
-        pa[0] = a1a;
-        pa[1] = s2a + s2b;
-    }
 }
 
 // TILES row blocks per thread block: every load of all tiles is issued before

@@ -1,0 +1,615 @@
+// rhs_turn.hpp -- the LV-ELVA attempt in two launches instead of three (or
+// five), for any even N = 2^a 3^b 5^c 7^d from 48 to 512.
+//
+//   kt_col    column pass: applies the previous attempt's accept / reject, then
+//             Hartley along y, divide by kappa R, Hartley along y   (g2 -> g1)
+//   kt_turn   turns one attempt into the next: Hartley along x of its own and
+//             its neighbours' rows, /N^2, corner BC, stage sums, error
+//             partials (g1 -> x'), and, on the new state while it is still on
+//             chip, the flexure stencil and the forward Hartley transform
+//             along x of the next attempt                           (x' -> g2)
+//
+// A round of launches begins with kt_turn(first), which only does the forward
+// part on the current state, and then alternates kt_col, kt_turn.
+//
+// Why: one domain's attempt is bound by its launches, not by bytes -- each
+// costs about 2 us before its first load returns, and every pass then waits
+// for descriptor, control block and fields in turn.  The stencil needs two
+// halo rows of the new state on each side, exactly one complex line (rows
+// 2j, 2j+1 share one), so a block of LO line pairs transforms LO + 2 and the
+// inverse pass, the stencil and the forward pass become one launch.
+//
+// The new state is assumed accepted (about 99 of 100 attempts are).  After a
+// rejection the right-hand side is unchanged -- it reads now%w -- and g1 still
+// holds it: kt_col does nothing and the next kt_turn repeats the stage sums
+// with the smaller step, so no attempt is lost.  An attempt that can end the
+// update (t + dt >= tf) skips the forward part.
+//
+// Arithmetic and reduction orders are those of the three-pass kernels
+// (rhs_fast.hip) where those exist, so a domain gives the same bits in a
+// small group here and in a large one there.
+#pragma once
+#include "fft_mix.hpp"
+#include "fi_kernels.h"
+#include "rhs_common.hpp"
+
+namespace fi {
+
+// lengths of the register kernels of rhs_fast.hip, whose error partials these
+// kernels reproduce: one per row pair, reduced over N/8 threads of 8 columns
+// (the other lengths: one per row, as the mixed-radix LDS kernels of rhs.hip)
+constexpr bool turn_reg8(int n) { return (n & (n - 1)) == 0 || n == 192 || n == 384; }
+
+template <typename T, int N, int LO> struct Turn {
+    using PL = MixPlan<N>;
+    static constexpr int LINES = LO + 2, ROWS = 2 * LO, WR = ROWS + 4;
+    static constexpr int need() {
+        int t = LINES * PL::TPL;
+        if (t < N) t = N;
+        return t;
+    }
+    static constexpr int THREADS = (need() + 63) / 64 * 64;
+    static constexpr int NB = (N / 2 + LO - 1) / LO;                        // blocks per domain
+    static constexpr size_t tw_bytes = (size_t)N * sizeof(cplx<T>);
+    static constexpr size_t x_bytes = (size_t)WR * N * sizeof(double);      // new state; later f
+    static constexpr size_t z_bytes = (size_t)2 * LINES * MixRow<T, N>::PITCH * sizeof(cplx<T>);
+    static constexpr size_t m_bytes = (size_t)(2 * ROWS + 2) * N * sizeof(double);
+    static constexpr size_t lds = tw_bytes + x_bytes + (z_bytes > m_bytes ? z_bytes : m_bytes);
+    static_assert(N % 2 == 0 && N >= ROWS, "domain smaller than a block");
+};
+
+template <typename T, int N, int LO, bool UNI>
+__global__ void __launch_bounds__((Turn<T, N, LO>::THREADS)) kt_turn(const Member* __restrict__ mem,
+                                                                   const void* __restrict__ twv, int first) {
+    using TN = Turn<T, N, LO>;
+    using PL = MixPlan<N>;
+    constexpr int THREADS = TN::THREADS, LINES = TN::LINES, ROWS = TN::ROWS, WR = TN::WR, TPL = PL::TPL, T0 = PL::T0;
+    constexpr bool REG8 = turn_reg8(N);
+    int mi, blk;
+    xcd_order(mi, blk);
+    const Member& M = mem[mi];
+    // the member's pointers in one batch of scalar loads
+    const Ctl* const p_ctl = first ? M.ctl : M.ctl_next;
+    const void *p_src = M.g1, *p_D = M.D, *p_C = M.cfull, *p_E = M.eta;
+    const double *p_cor = M.corners, *x0 = M.X[0], *x1p = M.X[1], *wW = M.W;
+    scalars_ready(p_ctl, p_src, p_D, p_C, p_E, p_cor, x0, x1p, wW);
+    extern __shared__ __align__(16) unsigned char smem[];
+    cplx<T>* tw_l = (cplx<T>*)smem;
+    double* xr = (double*)(smem + TN::tw_bytes);
+    unsigned char* zreg = smem + TN::tw_bytes + TN::x_bytes;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // rows [row0, row0 + ROWS); where the blocks do not divide the domain the
+    // last one reaches back over rows of the one before and leaves them to it
+    const int row0 = min(blk * ROWS, N - ROWS), own0 = blk * LO - row0 / 2;
+    const int col = tid < N ? tid : N - 1;
+    const int lane_line = tid / TPL, t = tid % TPL;
+    // global line (row pair) of local line li (0: the halo above), clamped
+    auto gline = [&](int li) {
+        const int g = row0 / 2 - 1 + li;
+        return g < 0 ? 0 : (g > N / 2 - 1 ? N / 2 - 1 : g);
+    };
+    auto crow = [](int r) { return r < 0 ? 0 : (r > N - 1 ? N - 1 : r); };
+
+    // ---- loads that need no control block, in the order of use
+    constexpr int TWQ = (2 * N + THREADS - 1) / THREADS;
+    T twr[TWQ];
+    {
+        gptr<T> g = gin<T>(twv);
+#pragma unroll
+        for (int k = 0; k < TWQ; ++k) twr[k] = g[min(tid + THREADS * k, 2 * N - 1)];
+    }
+    cplx<T> v[PL::E];
+    constexpr int NW = THREADS / 64, QPW = NW >= 4 ? 1 : (4 + NW - 1) / NW, CPL = (N + 63) / 64;
+    double cq[QPW][CPL];
+    if (!first) {
+        gptr<T> src = gin<T>(p_src);
+        const int g = gline(lane_line < LINES ? lane_line : 0), tt = t < T0 ? t : 0;
+#pragma unroll
+        for (int r = 0; r < PL::R0; ++r)
+            v[r] = mk<T>(src[(size_t)(2 * g) * N + tt + T0 * r], src[(size_t)(2 * g + 1) * N + tt + T0 * r]);
+        // the four corner sums over the column pass's N terms: quantity q by
+        // wave q (waves 4.. repeat 0..3; fewer waves take several), lane-strided
+        gptr<double> cp = gin<double>(p_cor);
+#pragma unroll
+        for (int j = 0; j < QPW; ++j) {
+            const int qi = NW >= 4 ? (wave & 3) : wave + NW * j;
+#pragma unroll
+            for (int k = 0; k < CPL; ++k) {
+                const int c = lane + 64 * k;
+                cq[j][k] = cp[(size_t)(c < N ? c : N - 1) * 4 + (qi & 3)];
+            }
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // rheology and load of the thread's column strip (D rows -1 .. ROWS)
+    T dv[ROWS + 2], cv[ROWS], ev[ROWS];
+    {
+        gptr<T> Dg = gin<T>(p_D), Cg = gin<T>(p_C), Eg = gin<T>(p_E);
+#pragma unroll
+        for (int r = 0; r < ROWS + 2; ++r) dv[r] = (Dg + (size_t)crow(row0 - 1 + r) * N)[col];
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            cv[r] = (Cg + (size_t)(row0 + r) * N)[col];
+            ev[r] = (Eg + (size_t)(row0 + r) * N)[col];
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const kptr<Ctl> c = kview(p_ctl);
+    const kptr<PhysDev> ph = kview(M.phys);
+    const bool run = c->status == ST_RUN;
+    const int cur = c->cur;
+#pragma unroll
+    for (int k = 0; k < TWQ; ++k)
+        if (tid + THREADS * k < 2 * N) ((T*)tw_l)[tid + THREADS * k] = twr[k];
+    // kt_col left the decided control block in ctl_next; block 0 makes it
+    // current (every block reads ctl_next) and marks this attempt's decision
+    // as pending, after its last load
+    auto commit = [&](bool pending) {
+        if (!first && blk == 0 && tid == 0) {
+            copy_ctl(M.ctl, c);
+            if (pending) M.ctl->pending = 1;
+        }
+    };
+    if (!run) {
+        commit(false);
+        return;
+    }
+    bool ends = false;
+    if (first) {
+        gptr<double> w = gin<double>(c->w_is_x ? (cur ? x1p : x0) : wW);
+        double wl[WR];
+#pragma unroll
+        for (int r = 0; r < WR; ++r) wl[r] = (w + (size_t)crow(row0 - 2 + r) * N)[col];
+        if (tid < N) {
+#pragma unroll
+            for (int r = 0; r < WR; ++r) xr[r * N + tid] = wl[r];
+        }
+        __syncthreads();
+    } else {
+        const int meth = ph->dt_method;
+        const double dt = attempt_dt(meth, c->dt, c->t, c->tf, ph->dt_max);
+        ends = !(c->t + dt < c->tf);
+        gptr<double> X = gin<double>(cur ? x1p : x0);
+        gmut<double> Xn = gout<double>((void*)(cur ? x0 : x1p));
+        gmut<double> dw = gout<double>(M.dwdt);
+        gmut<double> part = gout<double>(M.partials);
+        __shared__ double qs[4];
+        __shared__ double red[NW];
+        // the state, consumed after the transform: by line (8 columns of two
+        // rows per thread) or by column (all rows of the strip)
+        constexpr int TP8 = N / 8, XE = REG8 ? 16 : WR;
+        const int l8 = REG8 ? tid / TP8 : 0, t8 = REG8 ? tid % TP8 : 0;
+        const bool on8 = REG8 && l8 < LINES;
+        const int g8 = gline(on8 ? l8 : 0);
+        double xv[XE];
+        if constexpr (REG8) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                xv[2 * e] = X[(size_t)(2 * g8) * N + t8 + TP8 * e];
+                xv[2 * e + 1] = X[(size_t)(2 * g8 + 1) * N + t8 + TP8 * e];
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < WR; ++r) xv[r] = (X + (size_t)(2 * gline(r / 2) + (r & 1)) * N)[col];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < QPW; ++j) {
+            const int qi = NW >= 4 ? (wave & 3) : wave + NW * j;
+            double q = 0;
+#pragma unroll
+            for (int k = 0; k < CPL; ++k) q += lane + 64 * k < N ? cq[j][k] : 0.0;
+            q = wave_sum(q);
+            if (lane == 0 && qi < 4 && wave < 4) qs[qi] = q;
+        }
+        __syncthreads();
+        const bool on = lane_line < LINES;
+        MixRow<T, N> xc((cplx<T>*)zreg, LINES, on ? lane_line : 0);
+        mix_fft<T, N>(v, t, on, tw_l, xc);
+        // /(nx*ny*1.) (lv_elva.f90:117): an exact multiplication for N = 2^k
+        const double S = (double)(float)((double)N * (double)N), rS = 1.0 / S;
+        auto scl = [&](double x) {
+            if constexpr ((N & (N - 1)) == 0) return x * rS;
+            else return x / S;
+        };
+        // x(1,1) + x(nx,ny) + x(1,ny) + x(nx,1)  (isos_utils.f90:116)
+        const double cc = 0.25 * (scl(qs[0]) + scl(qs[3]) + scl(qs[2]) + scl(qs[1]));
+        const double spy = ph->sec_per_year;
+        // one cell: k, stage sums, statistics; the new state to LDS and, in
+        // the block's own lines, to memory
+        auto cell = [&](int r, int k, size_t at, bool own, T h, double x, double& a, double& s2) {
+            const double kk = (scl((double)h) - cc) * spy;
+            double x1;
+            const double x2 = stage_sums(meth, x, kk, dt, x1);
+            xr[r * N + k] = x2;
+            if (own) {
+                if (ends) dw[at] = kk;
+                Xn[at] = x2;
+            }
+            a = fmax(a, fmax(fabs(x1), fabs(x2)));
+            const double d = x2 - x1;
+            s2 += d * d;
+        };
+        if constexpr (REG8) {
+            double a = 0.0, s2a = 0.0, s2b = 0.0;
+            const bool own = on8 && l8 >= 1 + own0 && l8 <= LO;
+            if (on8) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int k = t8 + TP8 * e;
+                    T ha, hb;
+                    dht_pair(xc.at(l8, k), xc.at(l8, k ? N - k : 0), ha, hb);
+                    const size_t at = (size_t)(2 * g8) * N + k;
+                    cell(2 * l8, k, at, own, ha, xv[2 * e], a, s2a);
+                    cell(2 * l8 + 1, k, at + N, own, hb, xv[2 * e + 1], a, s2b);
+                }
+            }
+            row_reduce_store<TP8>(a, 0.0, s2a, 0.0, 0.0, s2b, on8 ? l8 : 0, on8 ? t8 : 1, part + (size_t)g8 * 4, own);
+            __syncthreads();
+        } else {
+            // partials per row, in the order of the mixed-radix LDS kernels
+            // (rhs.hip): lane l of a wave sums columns l, l + 64, ..., then a
+            // butterfly.  The squares go through the exchange's free buffer.
+            double* dd = (double*)((cplx<T>*)zreg + (xc.cur ^ 1) * xc.size);
+            static_assert((size_t)LINES * MixRow<T, N>::PITCH * sizeof(cplx<T>) >= (size_t)ROWS * N * sizeof(double),
+                          "squares of the block's rows fit one exchange buffer");
+            double a = 0.0;
+            if (tid < N) {
+#pragma unroll
+                for (int l = 0; l < LINES; ++l) {
+                    T ha, hb;
+                    dht_pair(xc.at(l, tid), xc.at(l, tid ? N - tid : 0), ha, hb);
+                    const bool inner = l >= 1 && l <= LO;
+                    const bool own = inner && l >= 1 + own0;
+                    const size_t at = (size_t)(2 * gline(l)) * N + tid;
+                    double am = 0.0, da = 0.0, db = 0.0;
+                    cell(2 * l, tid, at, own, ha, xv[2 * l], am, da);
+                    cell(2 * l + 1, tid, at + N, own, hb, xv[2 * l + 1], am, db);
+                    if (inner) {
+                        a = fmax(a, am);
+                        dd[(2 * l - 2) * N + tid] = da;
+                        dd[(2 * l - 1) * N + tid] = db;
+                    }
+                }
+            }
+            a = wave_max(a);
+            if (lane == 0) red[wave] = a;
+            __syncthreads();
+            for (int r = wave; r < ROWS; r += NW) {
+                double sm = 0.0;
+                for (int k = lane; k < N; k += 64) sm += dd[r * N + k];
+                sm = wave_sum(sm);
+                // (only the largest maximum of all partials is used: the
+                // block's stands for each of its rows)
+                double am = red[0];
+                for (int w = 1; w < NW; ++w) am = fmax(am, red[w]);
+                if (lane == 0 && r >= 2 * own0) {
+                    gmut<double> pp = part + (size_t)(row0 + r) * 4;
+                    pp[0] = am;
+                    pp[1] = sm;
+                }
+            }
+            __syncthreads();   // the squares' buffer is part of the stencil's
+        }
+        if (ends) {   // no next attempt if this one is accepted; after a rejection the next kt_turn comes back here
+            commit(true);
+            return;
+        }
+    }
+
+    // ---- stencil on the thread's column strip (formulas and operand order of
+    // rhs_fast.hip's march; one-sided windows at the domain edges)
+    const double nu = ph->nu, g = ph->g;
+    const double invq = ph->inv_dx2, inv1 = ph->inv_dx, inv2 = ph->inv_2dx;
+    const bool top = row0 == 0, bottom = row0 + ROWS == N;
+    double* sxx = (double*)zreg;                 // Mxx rows 0 .. ROWS-1
+    double* sxy = sxx + ROWS * N;                // Mxy rows -1 .. ROWS
+    const int ii = tid < 1 ? 1 : (tid > N - 2 ? N - 2 : tid);
+    const bool left = tid == 0, right = tid == N - 1;
+    double my[ROWS + 2];
+    // distortion: spacing of the strip's own column, and of the column the
+    // second x-difference divides by (the first one at the right edge,
+    // finite_differences.f90)
+    double h1[UNI ? 1 : WR], hq[UNI ? 1 : WR];
+    if constexpr (!UNI) {
+        gptr<double> dxm = gin<double>(M.dxm);
+#pragma unroll
+        for (int r = 0; r < WR; ++r) {
+            h1[r] = (dxm + (size_t)crow(row0 - 2 + r) * N)[col];
+            hq[r] = (dxm + (size_t)crow(row0 - 2 + r) * N)[right ? 0 : col];
+        }
+    }
+    // difference quotients of a in strip row r: centred / one-sided first, second
+    auto q1 = [&](double a, bool one, int r) {
+        if constexpr (UNI) return a * (one ? inv1 : inv2);
+        else return a / (one ? h1[r] : 2 * h1[r]);
+    };
+    auto qx = [&](double a, int r) {
+        if constexpr (UNI) return a * invq;
+        else return a / (hq[r] * hq[r]);
+    };
+    auto qy = [&](double a, int r) {
+        if constexpr (UNI) return a * invq;
+        else return a / (h1[r] * h1[r]);
+    };
+    if (tid < N) {
+        double wv[WR], wx[WR], wxx[WR];
+#pragma unroll
+        for (int r = 0; r < WR; ++r) {
+            const double* row = xr + r * N;
+            const double a = row[ii + 1], b = row[ii], d = row[ii - 1];
+            wv[r] = left ? d : (right ? a : b);
+            wx[r] = q1((left ? b : a) - (right ? b : d), left || right, r);
+            wxx[r] = qx(a - 2 * b + d, r);
+        }
+#pragma unroll
+        for (int m = -1; m <= ROWS; ++m) {
+            const int r = m + 2;
+            double wa = wv[r + 1], wb = wv[r], wc = wv[r - 1];
+            double whi = wx[r + 1], wlo = wx[r - 1];
+            bool one = false;
+            if (m == 0 && top) { wa = wv[4]; wb = wv[3]; wc = wv[2]; wlo = wx[2]; one = true; }
+            if (m == ROWS - 1 && bottom) {
+                wa = wv[ROWS + 1]; wb = wv[ROWS]; wc = wv[ROWS - 1]; whi = wx[ROWS + 1];
+                one = true;
+            }
+            const double wyy = qy(wa - 2 * wb + wc, r);
+            const double wxy = q1(whi - wlo, one, r);
+            const double D = (double)dv[m + 1];
+            if (m >= 0 && m < ROWS) sxx[m * N + tid] = -(D * (wxx[r] + nu * wyy));
+            my[m + 1] = -(D * (wyy + nu * wxx[r]));
+            sxy[(m + 1) * N + tid] = -(D * (1.0 - nu) * wxy);
+        }
+    }
+    __syncthreads();
+    T* sf = (T*)xr;   // the state rows have been read
+    if (tid < N) {
+        double mx[ROWS + 2];
+#pragma unroll
+        for (int r = 0; r < ROWS + 2; ++r) {
+            const double* row = sxy + r * N;
+            mx[r] = q1(row[right ? tid : tid + 1] - row[left ? tid : tid - 1], left || right, r + 1);
+        }
+#pragma unroll
+        for (int j = 0; j < ROWS; ++j) {
+            const double* xrow = sxx + j * N;
+            const double mxx = qx(xrow[ii + 1] - 2 * xrow[ii] + xrow[ii - 1], j + 2);
+            double ya = my[j + 2], yb = my[j + 1], yc = my[j];
+            double hi = mx[j + 2], lo = mx[j];
+            bool one = false;
+            if (j == 0 && top) { ya = my[3]; yb = my[2]; yc = my[1]; lo = mx[1]; one = true; }
+            if (j == ROWS - 1 && bottom) {
+                ya = my[ROWS]; yb = my[ROWS - 1]; yc = my[ROWS - 2]; hi = mx[ROWS];
+                one = true;
+            }
+            const double myy = qy(ya - 2 * yb + yc, j + 2);
+            const double mxyxy = q1(hi - lo, one, j + 2);
+            const double p = -(g * (double)cv[j]);
+            const double num = p + mxx + 2.0 * mxyxy + myy;
+            T f;
+            if constexpr (sizeof(T) == 8) f = (T)(num / (2.0 * (double)ev[j]));
+            else f = (T)(num * (double)ev[j]);   // mixed: eta holds 1/(2 eta)
+            sf[j * N + tid] = f;
+        }
+    }
+    __syncthreads();
+
+    // ---- forward row transform of the block's own lines
+    {
+        const bool on = lane_line < LO;
+        const int l = on ? lane_line : 0;
+        if (on && t < T0) {
+#pragma unroll
+            for (int r = 0; r < PL::R0; ++r)
+                v[r] = mk<T>(sf[2 * l * N + t + T0 * r], sf[(2 * l + 1) * N + t + T0 * r]);
+        }
+        MixRow<T, N> xc((cplx<T>*)zreg, LINES, l);
+        mix_fft<T, N>(v, t, on, tw_l, xc);
+        gmut<T> dst = gout<T>(M.g2);
+        if (tid < N) {
+#pragma unroll
+            for (int p = 0; p < LO; ++p) {
+                T ha, hb;
+                dht_pair(xc.at(p, tid), xc.at(p, tid ? N - tid : 0), ha, hb);
+                if (p >= own0) {
+                    const size_t at = (size_t)(row0 + 2 * p) * N + tid;
+                    dst[at] = ha;
+                    dst[at + N] = hb;
+                }
+            }
+        }
+    }
+    commit(true);
+}
+
+// Column pass.  C complex lines (columns 2j, 2j+1) per block; the last block
+// of a domain transforms copies of its last line where C does not divide N/2.
+template <typename T, int N, int C> struct TurnCol {
+    static constexpr int THREADS = (C * MixPlan<N>::TPL + 63) / 64 * 64;
+    static constexpr int NB = (N / 2 + C - 1) / C;
+    static constexpr size_t lds = ((size_t)N + 2 * (size_t)MixCol<T, N, C>::SIZE) * sizeof(cplx<T>);
+};
+
+template <typename T, int N, int C>
+__global__ void __launch_bounds__((TurnCol<T, N, C>::THREADS)) kt_col(const Member* __restrict__ mem,
+                                                                    const void* __restrict__ twv,
+                                                                    const double2* __restrict__ tw64) {
+    using PL = MixPlan<N>;
+    constexpr int THREADS = TurnCol<T, N, C>::THREADS, R0 = PL::R0, T0 = PL::T0;
+    // a domain's column blocks on one XCD: neighbours share 128-byte lines
+    int mi, cblk;
+    xcd_order(mi, cblk);
+    const Member& M = mem[mi];
+    const void *p_src = M.g2, *p_kr = M.kR;
+    const Ctl* const p_ctl = M.ctl;
+    const double* const p_part = M.partials;
+    scalars_ready(p_src, p_kr, p_ctl, p_part);
+    extern __shared__ __align__(16) unsigned char smem[];
+    cplx<T>* tw_l = (cplx<T>*)smem;
+    const int tid = threadIdx.x, line = tid % C, t = tid / C;
+    const bool live = cblk * C + line < N / 2, on = t < PL::TPL;
+    const int ca = 2 * (live ? cblk * C + line : N / 2 - 1), tt = t < T0 ? t : 0;
+    // the previous attempt's partials first (the decision needs them), then
+    // twiddles, spectrum and kappa R; none of them depends on the control block
+    constexpr int NP = turn_reg8(N) ? N / 2 : N, PJ = (NP + 63) / 64;
+    double pa[PJ][2];
+    {
+        gptr<double> part = gin<double>(p_part);
+        const int lane = tid & 63;
+#pragma unroll
+        for (int j = 0; j < PJ; ++j) {
+            const int b = lane + 64 * j < NP ? lane + 64 * j : NP - 1;
+#pragma unroll
+            for (int k = 0; k < 2; ++k) pa[j][k] = part[(size_t)b * 4 + k];
+        }
+    }
+    constexpr int TWQ = (2 * N + THREADS - 1) / THREADS;
+    T twr[TWQ];
+    {
+        gptr<T> g = gin<T>(twv);
+#pragma unroll
+        for (int k = 0; k < TWQ; ++k) twr[k] = g[min(tid + THREADS * k, 2 * N - 1)];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    using V2 = typename vec2<T>::type;
+    gptr<V2> src = gin<V2>(p_src), kR = gin<V2>(p_kr);
+    // (row, column pair) -> vector index
+    auto vec = [&](int row) { return ((unsigned)row * N + ca) / 2; };
+    V2 xs[R0], xk[R0];
+#pragma unroll
+    for (int r = 0; r < R0; ++r) xs[r] = src[vec(tt + T0 * r)];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < R0; ++r) xk[r] = kR[vec(tt + T0 * r)];
+    const double2 wa = tw64[ca], wb = tw64[ca + 1];
+    __builtin_amdgcn_sched_barrier(0);
+    const kptr<Ctl> c = kview(p_ctl);
+    StepState st = load_state(c);
+    const bool pending = c->pending != 0;
+#pragma unroll
+    for (int k = 0; k < TWQ; ++k)
+        if (tid + THREADS * k < 2 * N) ((T*)tw_l)[tid + THREADS * k] = twr[k];
+    // block 0 writes the decided control block to ctl_next, which kt_turn
+    // reads and makes current; every block decides alike
+    auto write_next = [&]() {
+        if (cblk == 0 && tid == 0) {
+            copy_ctl(M.ctl_next, c);
+            store_state(M.ctl_next, st);
+            M.ctl_next->pending = 0;
+            M.ctl_next->skip = 0;
+        }
+    };
+    bool go = st.status == ST_RUN;
+    if (pending) {
+        const int lane = tid & 63;
+        double amax = 0.0, s2 = 0.0;
+#pragma unroll
+        for (int j = 0; j < PJ; ++j) {
+            const bool in = lane + 64 * j < NP;
+            amax = fmax(amax, in ? pa[j][0] : 0.0);
+            s2 += in ? pa[j][1] : 0.0;
+        }
+        amax = wave_max(amax);
+        s2 = wave_sum(s2);
+        const long long acc = st.accepts;
+        st = decide_step(st, amax, s2, kview(M.phys), N);
+        // a rejected attempt keeps its right-hand side: g1 holds it
+        go = __builtin_amdgcn_readfirstlane(st.status == ST_RUN && st.accepts != acc);
+    }
+    if (!go) {
+        write_next();
+        return;
+    }
+    cplx<T> v[PL::E];
+#pragma unroll
+    for (int r = 0; r < R0; ++r) v[r] = mk<T>(xs[r].x, xs[r].y);
+    __syncthreads();
+    MixCol<T, N, C> xc((cplx<T>*)smem + N, line);
+    mix_fft<T, N>(v, t, on, tw_l, xc);
+    const bool has = on && t < T0;
+    if (has) {
+        // Hartley values and the spectral divide (lv_elva.f90:115)
+#pragma unroll
+        for (int r = 0; r < R0; ++r) {
+            const int k = t + T0 * r;
+            T ha, hb;
+            dht_pair(xc.get(k), xc.get(k ? N - k : 0), ha, hb);
+            v[r] = mk<T>(kdiv(ha, xk[r].x), kdiv(hb, xk[r].y));
+        }
+    }
+    xc.flip();
+    mix_fft<T, N>(v, t, on, tw_l, xc);
+    if (has && live) {
+        gmut<V2> dst = gout<V2>(M.g1);
+        gmut<double> cor = gout<double>(M.corners);
+#pragma unroll
+        for (int r = 0; r < R0; ++r) {
+            const int k = t + T0 * r;
+            T ha, hb;
+            dht_pair(xc.get(k), xc.get(k ? N - k : 0), ha, hb);
+            V2 o;
+            o.x = ha;
+            o.y = hb;
+            dst[vec(k)] = o;
+            // per-column terms of the four corners of the inverse transform
+            // (rows 0 and N-1, weights 1 and cas(2 pi col (N-1) / N))
+            if (k == 0 || k == N - 1) {
+                const int q = (k == 0) ? 0 : 2;
+                const double va = (double)ha, vb = (double)hb;
+                cor[(size_t)ca * 4 + q] = va;
+                cor[(size_t)ca * 4 + q + 1] = va * (wa.x + wa.y);
+                cor[(size_t)(ca + 1) * 4 + q] = vb;
+                cor[(size_t)(ca + 1) * 4 + q + 1] = vb * (wb.x + wb.y);
+            }
+        }
+    }
+    write_next();
+}
+
+// ------------------------------------------------------------------ launchers
+// LDS of one workgroup on gfx950; above 64 KiB it is declared to the runtime
+template <class K> bool turn_lds_ok(K kern, size_t lds) {
+    if (lds > 160 * 1024) return false;
+    return lds <= 65536 || hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               (int)lds) == hipSuccess;
+}
+
+template <typename T, int N, int LO, bool UNI>
+bool turn_rows(const Member* d, int nmem, const RhsShape& s, hipStream_t st, int which) {
+    using TN = Turn<T, N, LO>;
+    static const bool ok = turn_lds_ok(kt_turn<T, N, LO, UNI>, TN::lds);
+    if (!ok || which < 0) return ok;
+    const bool first = which == 0;
+    launch_k(first ? 0 : 3, kt_turn<T, N, LO, UNI>, dim3(TN::NB, nmem), dim3(TN::THREADS), TN::lds, st, d, s.tw,
+             first ? 1 : 0);
+    return true;
+}
+template <typename T, int N, int C>
+bool turn_cols(const Member* d, int nmem, const RhsShape& s, hipStream_t st, int which) {
+    using TC = TurnCol<T, N, C>;
+    static const bool ok = turn_lds_ok(kt_col<T, N, C>, TC::lds);
+    if (!ok || which < 0) return ok;
+    launch_k(2, kt_col<T, N, C>, dim3(TC::NB, nmem), dim3(TC::THREADS), TC::lds, st, d, s.tw, s.tw64);
+    return true;
+}
+
+template <typename T, int N>
+bool turn_n(const Member* d, int nmem, const RhsShape& s, hipStream_t st, int which) {
+    const bool cols = which == 1 || which < 0, rows = which != 1;
+    bool ok = true;
+    if (cols) ok = s.turn_C >= 8 ? turn_cols<T, N, 8>(d, nmem, s, st, which) : turn_cols<T, N, 2>(d, nmem, s, st, which);
+    if (rows && ok)
+        ok = s.uniform ? (s.turn_LO == 1 ? turn_rows<T, N, 1, true>(d, nmem, s, st, which)
+                                         : turn_rows<T, N, 2, true>(d, nmem, s, st, which))
+                       : turn_rows<T, N, 2, false>(d, nmem, s, st, which);
+    return ok;
+}
+
+template <int... Ns>
+TurnFn turn_lookup(int n, bool fp64) {
+    TurnFn f = nullptr;
+    ((n == Ns ? (void)(f = fp64 ? turn_n<double, Ns> : turn_n<float, Ns>) : (void)0), ...);
+    return f;
+}
+
+}  // namespace fi
