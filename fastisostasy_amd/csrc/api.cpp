@@ -385,19 +385,21 @@ int make_three_pass_shape(int n, int nmem, bool fp64, bool uniform, bool tuned, 
 
 // Two-launch attempts (rhs_turn.hpp) for this group?  At the general lengths
 // always: they replace five launches of the mixed-radix LDS kernels (one
-// N = 320 domain, mixed: 17.1 us per attempt against 59.5; 64 of 200^2: 62.5
+// N = 320 domain, mixed: 16.4 us per attempt against 59.5; 64 of 200^2: 60.5
 // against 155).  At the lengths of the three-launch register kernels (2^k,
-// 3 * 2^k) only for small groups that those serve with five launches: distorted
-// grids and N = 192 (uniform N = 192: 17.5 us against 26.9; uniform N = 256 is
-// a tie, 16.9 against 17.1).  A launch shape asked of the other kernels
-// (environment, autotuner) keeps those; FI_TURN = 0 never, 2 wherever the
-// kernels exist (tests).
+// 3 * 2^k) while launches and not bytes set the pace, measured per attempt
+// (two launches against three, mixed): one 64^2 domain 12.9 / 16.0 us, 256^2
+// 14.1 / 16.9, 512^2 17.9 / 19.8; 48 of 128^2 21.3 / 23.8, 12 of 256^2 23.0 /
+// 23.7 but 16 27.2 / 25.3; 6 of 384^2 31.1 / 35.5; 2 of 512^2 20.3 / 21.5 but 3
+// 29.8 / 26.8 and 2 in FP64 27.5 / 26.1.  A launch shape asked of the other
+// kernels (environment, autotuner) keeps those; FI_TURN = 0 never, 2 wherever
+// the kernels exist (tests).
 //
-// Blocks: one line pair per kt_turn block while two would leave CUs idle (N =
-// 320: 17.1 us against 18.7; 30 of 200^2: 39 against 49 the other way round),
-// 2 line pairs per kt_col block until 8 give every CU a block (30 of 200^2:
-// 39.4 us per attempt against 45.1).
-constexpr long long TURN_SMALL = 512;   // blocks of two line pairs
+// Blocks: one line pair per kt_turn block and two per kt_col block while that
+// leaves CUs idle otherwise (one N = 320 domain 16.4 us against 17.8 with 8
+// per kt_col block), from 192 blocks on two and eight (2 of 512^2: 20.3 us
+// against 25.6; 8 of 320^2: 28.9 against 32.6).
+long long turn_cells(int n, bool fp64) { return n < 512 ? 12 << 16 : fp64 ? 1 << 18 : 1 << 19; }
 
 void turn_shape(int n, int nmem, bool fp64, bool uniform, bool tuned, const TunedShape& ts, RhsShape& s) {
     s.turn = nullptr;
@@ -410,9 +412,12 @@ void turn_shape(int n, int nmem, bool fp64, bool uniform, bool tuned, const Tune
     if (want == 0) return;
     if (tuned && (ts.threads_row || ts.C || ts.row_tiles || ts.gL || ts.gC || ts.srow_rows || ts.threads_inv)) return;
     const long long blocks = (long long)(n / 4) * nmem;
-    if (s.fast && want != 2 && ((uniform && n != 192) || blocks > TURN_SMALL)) return;
-    s.turn_C = blocks >= 1024 ? 8 : 2;
-    s.turn_LO = blocks >= 256 ? 2 : 1;
+    if (s.fast && want != 2 && (long long)n * n * nmem > turn_cells(n, fp64)) return;
+    s.turn_C = blocks >= 192 ? 8 : 2;
+    s.turn_LO = blocks >= 192 ? 2 : 1;
+    // FI_TURN_LO = 1 | 2, FI_TURN_C = 2 | 8 override the blocks (tuning)
+    if (const char* e = std::getenv("FI_TURN_LO")) s.turn_LO = std::atoi(e) == 1 ? 1 : 2;
+    if (const char* e = std::getenv("FI_TURN_C")) s.turn_C = std::atoi(e) == 8 ? 8 : 2;
     TurnFn f = turn_find(n, fp64);
     // (a device that refuses the kernels' LDS keeps the others)
     if (f && f(nullptr, nmem, s, nullptr, -1)) s.turn = f;

@@ -77,6 +77,9 @@ template <int N> struct MixPlan {
         return t;
     }
     static constexpr int E = emax(), TPL = tpl();
+    // the first group reads no twiddles (a single stage): the table need not
+    // be published before the first exchange's barrier does so
+    static constexpr bool PLAIN0 = S.first[1] - S.first[0] == 1 && S.ng > 1;
     static constexpr int product(int a, int b) { return a >= b ? 1 : S.rad[a] * product(a + 1, b); }
 };
 
@@ -157,9 +160,10 @@ template <typename T, int N, int C> struct MixCol {
 // t + (N/R) r of the group's input (threads t < N/R).  Exit: the transform lies
 // in the exchange's current buffer, published by a barrier; the caller reads
 // it and flips the buffers before the next use.  Every thread of the block
-// must call (on: the thread has a line).
-template <typename T, int N, int G, class X>
-__device__ __forceinline__ void mix_fft_from(cplx<T>* v, int t, bool on, const cplx<T>* __restrict__ tw, X& xc) {
+// must call (on: the thread has a line).  last() runs before the last barrier.
+template <typename T, int N, int G, class X, class F>
+__device__ __forceinline__ void mix_fft_from(cplx<T>* v, int t, bool on, const cplx<T>* __restrict__ tw, X& xc,
+                                             F&& last) {
     using PL = MixPlan<N>;
     constexpr int R = PL::S.prod[G], NS = PL::S.ns[G], TG = N / R;
     if (on && (TG == PL::TPL || t < TG)) {
@@ -169,6 +173,7 @@ __device__ __forceinline__ void mix_fft_from(cplx<T>* v, int t, bool on, const c
 #pragma unroll
         for (int o = 0; o < R; ++o) xc.put(base + o * NS, v[o]);
     }
+    if constexpr (G + 1 == PL::NG) last();
     __syncthreads();
     if constexpr (G + 1 < PL::NG) {
         constexpr int RN = PL::S.prod[G + 1], TN = N / RN;
@@ -177,12 +182,16 @@ __device__ __forceinline__ void mix_fft_from(cplx<T>* v, int t, bool on, const c
             for (int r = 0; r < RN; ++r) v[r] = xc.get(t + TN * r);
         }
         xc.flip();
-        mix_fft_from<T, N, G + 1>(v, t, on, tw, xc);
+        mix_fft_from<T, N, G + 1>(v, t, on, tw, xc, last);
     }
+}
+template <typename T, int N, class X, class F>
+__device__ __forceinline__ void mix_fft(cplx<T>* v, int t, bool on, const cplx<T>* __restrict__ tw, X& xc, F&& last) {
+    mix_fft_from<T, N, 0>(v, t, on, tw, xc, last);
 }
 template <typename T, int N, class X>
 __device__ __forceinline__ void mix_fft(cplx<T>* v, int t, bool on, const cplx<T>* __restrict__ tw, X& xc) {
-    mix_fft_from<T, N, 0>(v, t, on, tw, xc);
+    mix_fft_from<T, N, 0>(v, t, on, tw, xc, [] {});
 }
 
 }  // namespace fi

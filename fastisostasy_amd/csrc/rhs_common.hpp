@@ -183,6 +183,21 @@ __device__ __forceinline__ StepState decide_step(StepState s, double amax, doubl
     return s;
 }
 
+// Whether decide_step would accept the attempt and leave the update running.
+// sqrt is monotone and exact at 1, so err < 1 without the root.
+__device__ __forceinline__ bool step_goes_on(double c_dt, double c_t, double c_tf, double amax, double s2,
+                                             const kptr<PhysDev> ph, int n) {
+    const int m = ph->dt_method;
+    const double dt = attempt_dt(m, c_dt, c_t, c_tf, ph->dt_max);
+    bool accept = true;
+    if (m == 2 || m == 3) {
+        const double tol = ph->atol + ph->rtol * amax;
+        const double nn = (double)n * (double)n;
+        accept = s2 / (tol * tol) / nn < 1;
+    }
+    return accept && c_t + dt < c_tf;
+}
+
 // Field-wise copy of a control block read through the scalar cache.
 __device__ __forceinline__ void copy_ctl(Ctl* d, const kptr<Ctl> s) {
     d->t = s->t; d->dt = s->dt; d->tf = s->tf; d->err = s->err; d->tol = s->tol;

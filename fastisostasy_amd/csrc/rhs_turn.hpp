@@ -54,7 +54,9 @@ template <typename T, int N, int LO> struct Turn {
     static constexpr size_t x_bytes = (size_t)WR * N * sizeof(double);      // new state; later f
     static constexpr size_t z_bytes = (size_t)2 * LINES * MixRow<T, N>::PITCH * sizeof(cplx<T>);
     static constexpr size_t m_bytes = (size_t)(2 * ROWS + 2) * N * sizeof(double);
-    static constexpr size_t lds = tw_bytes + x_bytes + (z_bytes > m_bytes ? z_bytes : m_bytes);
+    static constexpr size_t d_bytes = (size_t)ROWS * N * sizeof(double);    // squared errors
+    static constexpr size_t zm_bytes = z_bytes > m_bytes ? z_bytes : m_bytes;
+    static constexpr size_t lds = tw_bytes + x_bytes + zm_bytes + d_bytes;
     static_assert(N % 2 == 0 && N >= ROWS, "domain smaller than a block");
 };
 
@@ -73,10 +75,17 @@ __global__ void __launch_bounds__((Turn<T, N, LO>::THREADS)) kt_turn(const Membe
     const void *p_src = M.g1, *p_D = M.D, *p_C = M.cfull, *p_E = M.eta;
     const double *p_cor = M.corners, *x0 = M.X[0], *x1p = M.X[1], *wW = M.W;
     scalars_ready(p_ctl, p_src, p_D, p_C, p_E, p_cor, x0, x1p, wW);
+    // the control block and physics scalars, in flight while the vector loads
+    // are issued
+    const kptr<Ctl> c = kview(p_ctl);
+    const kptr<PhysDev> ph = kview(M.phys);
+    const int status = c->status, cur = c->cur, w_is_x = c->w_is_x, meth = ph->dt_method;
+    const double c_dt = c->dt, c_t = c->t, c_tf = c->tf, dt_max = ph->dt_max, spy = ph->sec_per_year;
     extern __shared__ __align__(16) unsigned char smem[];
     cplx<T>* tw_l = (cplx<T>*)smem;
     double* xr = (double*)(smem + TN::tw_bytes);
     unsigned char* zreg = smem + TN::tw_bytes + TN::x_bytes;
+    double* dd = (double*)(zreg + TN::zm_bytes);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // rows [row0, row0 + ROWS); where the blocks do not divide the domain the
     // last one reaches back over rows of the one before and leaves them to it
@@ -134,10 +143,7 @@ __global__ void __launch_bounds__((Turn<T, N, LO>::THREADS)) kt_turn(const Membe
         }
     }
     __builtin_amdgcn_sched_barrier(0);
-    const kptr<Ctl> c = kview(p_ctl);
-    const kptr<PhysDev> ph = kview(M.phys);
-    const bool run = c->status == ST_RUN;
-    const int cur = c->cur;
+    const bool run = status == ST_RUN;
 #pragma unroll
     for (int k = 0; k < TWQ; ++k)
         if (tid + THREADS * k < 2 * N) ((T*)tw_l)[tid + THREADS * k] = twr[k];
@@ -155,8 +161,70 @@ __global__ void __launch_bounds__((Turn<T, N, LO>::THREADS)) kt_turn(const Membe
         return;
     }
     bool ends = false;
+    __shared__ double qs[4];
+    __shared__ double red[NW];        // largest |x1|, |x2| of each wave
+    __shared__ double rg[LO][3][2];   // squared errors of a line's two rows, by lane group
+    // Error partials of the block's rows from their squares in dd, by the
+    // block's last waves, in the order of the other attempt kernels.  At the
+    // register kernels' lengths one entry per row pair: 8 columns per thread,
+    // a butterfly over groups of lanes, the groups in order; else one per row:
+    // lane l sums columns l, l + 64, ..., then a butterfly.  Only the largest
+    // of all the maxima is used: the block's stands for each of its entries.
+    constexpr int TP8 = REG8 ? N / 8 : 64, NG8 = (TP8 & (TP8 - 1)) == 0 ? 1 : 3, GL = TP8 / NG8;
+    auto block_max = [&]() {
+        double am = red[0];
+        for (int w = 1; w < NW; ++w) am = fmax(am, red[w]);
+        return am;
+    };
+    auto partials_sum = [&]() {   // after the barrier behind the squares
+        if constexpr (REG8) {
+            constexpr int W0 = NW - (LO * TP8 + 63) / 64;
+            const int q = tid - 64 * W0, l = q / TP8, t8 = q - l * TP8;
+            if (wave >= W0) {
+                const int lr = l < LO ? l : 0;
+                double sa[8], sb[8], s2a = 0.0, s2b = 0.0;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    sa[e] = dd[(2 * lr) * N + t8 + TP8 * e];
+                    sb[e] = dd[(2 * lr + 1) * N + t8 + TP8 * e];
+                }
+#pragma unroll
+                for (int e = 0; e < 8; ++e) { s2a += sa[e]; s2b += sb[e]; }
+                s2a = lanes_sum<GL>(s2a);
+                s2b = lanes_sum<GL>(s2b);
+                if (l < LO && t8 % GL == 0) { rg[l][t8 / GL][0] = s2a; rg[l][t8 / GL][1] = s2b; }
+            }
+        } else {
+            for (int r = NW - 1 - wave; r < ROWS; r += NW) {
+                double q[CPL], sm = 0.0;
+#pragma unroll
+                for (int k = 0; k < CPL; ++k) q[k] = dd[r * N + min(lane + 64 * k, N - 1)];
+#pragma unroll
+                for (int k = 0; k < CPL; ++k) sm += lane + 64 * k < N ? q[k] : 0.0;
+                sm = wave_sum(sm);
+                if (lane == 0 && r >= 2 * own0) {
+                    gmut<double> pp = gout<double>(M.partials) + (size_t)(row0 + r) * 4;
+                    pp[0] = block_max();
+                    pp[1] = sm;
+                }
+            }
+        }
+    };
+    auto partials_store = [&]() {   // after another barrier
+        if constexpr (REG8) {
+            const int l = THREADS - 1 - tid;
+            if (l < LO && l >= own0) {
+                double s2a = rg[l][0][0], s2b = rg[l][0][1];
+#pragma unroll
+                for (int w = 1; w < NG8; ++w) { s2a += rg[l][w][0]; s2b += rg[l][w][1]; }
+                gmut<double> pp = gout<double>(M.partials) + (size_t)(row0 / 2 + l) * 4;
+                pp[0] = block_max();
+                pp[1] = s2a + s2b;
+            }
+        }
+    };
     if (first) {
-        gptr<double> w = gin<double>(c->w_is_x ? (cur ? x1p : x0) : wW);
+        gptr<double> w = gin<double>(w_is_x ? (cur ? x1p : x0) : wW);
         double wl[WR];
 #pragma unroll
         for (int r = 0; r < WR; ++r) wl[r] = (w + (size_t)crow(row0 - 2 + r) * N)[col];
@@ -166,46 +234,30 @@ __global__ void __launch_bounds__((Turn<T, N, LO>::THREADS)) kt_turn(const Membe
         }
         __syncthreads();
     } else {
-        const int meth = ph->dt_method;
-        const double dt = attempt_dt(meth, c->dt, c->t, c->tf, ph->dt_max);
-        ends = !(c->t + dt < c->tf);
+        const double dt = attempt_dt(meth, c_dt, c_t, c_tf, dt_max);
+        ends = !(c_t + dt < c_tf);
         gptr<double> X = gin<double>(cur ? x1p : x0);
         gmut<double> Xn = gout<double>((void*)(cur ? x0 : x1p));
         gmut<double> dw = gout<double>(M.dwdt);
-        gmut<double> part = gout<double>(M.partials);
-        __shared__ double qs[4];
-        __shared__ double red[NW];
-        // the state, consumed after the transform: by line (8 columns of two
-        // rows per thread) or by column (all rows of the strip)
-        constexpr int TP8 = N / 8, XE = REG8 ? 16 : WR;
-        const int l8 = REG8 ? tid / TP8 : 0, t8 = REG8 ? tid % TP8 : 0;
-        const bool on8 = REG8 && l8 < LINES;
-        const int g8 = gline(on8 ? l8 : 0);
-        double xv[XE];
-        if constexpr (REG8) {
+        // the state of the thread's column, consumed after the transform
+        double xv[WR];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                xv[2 * e] = X[(size_t)(2 * g8) * N + t8 + TP8 * e];
-                xv[2 * e + 1] = X[(size_t)(2 * g8 + 1) * N + t8 + TP8 * e];
-            }
-        } else {
-#pragma unroll
-            for (int r = 0; r < WR; ++r) xv[r] = (X + (size_t)(2 * gline(r / 2) + (r & 1)) * N)[col];
-        }
+        for (int r = 0; r < WR; ++r) xv[r] = (X + (size_t)(2 * gline(r / 2) + (r & 1)) * N)[col];
         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int j = 0; j < QPW; ++j) {
-            const int qi = NW >= 4 ? (wave & 3) : wave + NW * j;
-            double q = 0;
-#pragma unroll
-            for (int k = 0; k < CPL; ++k) q += lane + 64 * k < N ? cq[j][k] : 0.0;
-            q = wave_sum(q);
-            if (lane == 0 && qi < 4 && wave < 4) qs[qi] = q;
-        }
-        __syncthreads();
+        if constexpr (!PL::PLAIN0) __syncthreads();
         const bool on = lane_line < LINES;
         MixRow<T, N> xc((cplx<T>*)zreg, LINES, on ? lane_line : 0);
-        mix_fft<T, N>(v, t, on, tw_l, xc);
+        mix_fft<T, N>(v, t, on, tw_l, xc, [&]() {
+#pragma unroll
+            for (int j = 0; j < QPW; ++j) {
+                const int qi = NW >= 4 ? (wave & 3) : wave + NW * j;
+                double q = 0;
+#pragma unroll
+                for (int k = 0; k < CPL; ++k) q += lane + 64 * k < N ? cq[j][k] : 0.0;
+                q = wave_sum(q);
+                if (lane == 0 && qi < 4 && wave < 4) qs[qi] = q;
+            }
+        });
         // /(nx*ny*1.) (lv_elva.f90:117): an exact multiplication for N = 2^k
         const double S = (double)(float)((double)N * (double)N), rS = 1.0 / S;
         auto scl = [&](double x) {
@@ -214,84 +266,64 @@ __global__ void __launch_bounds__((Turn<T, N, LO>::THREADS)) kt_turn(const Membe
         };
         // x(1,1) + x(nx,ny) + x(1,ny) + x(nx,1)  (isos_utils.f90:116)
         const double cc = 0.25 * (scl(qs[0]) + scl(qs[3]) + scl(qs[2]) + scl(qs[1]));
-        const double spy = ph->sec_per_year;
-        // one cell: k, stage sums, statistics; the new state to LDS and, in
-        // the block's own lines, to memory
-        auto cell = [&](int r, int k, size_t at, bool own, T h, double x, double& a, double& s2) {
-            const double kk = (scl((double)h) - cc) * spy;
-            double x1;
-            const double x2 = stage_sums(meth, x, kk, dt, x1);
-            xr[r * N + k] = x2;
-            if (own) {
-                if (ends) dw[at] = kk;
-                Xn[at] = x2;
-            }
-            a = fmax(a, fmax(fabs(x1), fabs(x2)));
-            const double d = x2 - x1;
-            s2 += d * d;
-        };
-        if constexpr (REG8) {
-            double a = 0.0, s2a = 0.0, s2b = 0.0;
-            const bool own = on8 && l8 >= 1 + own0 && l8 <= LO;
-            if (on8) {
+        // k, stage sums and statistics of C cells of the new state: all
+        // transform values first, then the arithmetic (the integrator's
+        // branch outside the cells), then the stores
+        //   h, x: transform value and state;  x2, d2: new state, squared error
+        auto cells = [&](auto cc_, const T* h, const double* x, double* kk, double* x2, double* d2, double& a) {
+            constexpr int C = decltype(cc_)::value;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int k = t8 + TP8 * e;
-                    T ha, hb;
-                    dht_pair(xc.at(l8, k), xc.at(l8, k ? N - k : 0), ha, hb);
-                    const size_t at = (size_t)(2 * g8) * N + k;
-                    cell(2 * l8, k, at, own, ha, xv[2 * e], a, s2a);
-                    cell(2 * l8 + 1, k, at + N, own, hb, xv[2 * e + 1], a, s2b);
+            for (int q = 0; q < C; ++q) kk[q] = (scl((double)h[q]) - cc) * spy;
+            auto sums = [&](auto mc) {
+#pragma unroll
+                for (int q = 0; q < C; ++q) {
+                    double x1;
+                    if constexpr (decltype(mc)::value == 3) x2[q] = stage_sums_m<3>(x[q], kk[q], dt, x1);
+                    else x2[q] = stage_sums(meth, x[q], kk[q], dt, x1);
+                    a = fmax(a, fmax(fabs(x1), fabs(x2[q])));
+                    const double d = x2[q] - x1;
+                    d2[q] = d * d;
                 }
-            }
-            row_reduce_store<TP8>(a, 0.0, s2a, 0.0, 0.0, s2b, on8 ? l8 : 0, on8 ? t8 : 1, part + (size_t)g8 * 4, own);
-            __syncthreads();
-        } else {
-            // partials per row, in the order of the mixed-radix LDS kernels
-            // (rhs.hip): lane l of a wave sums columns l, l + 64, ..., then a
-            // butterfly.  The squares go through the exchange's free buffer.
-            double* dd = (double*)((cplx<T>*)zreg + (xc.cur ^ 1) * xc.size);
-            static_assert((size_t)LINES * MixRow<T, N>::PITCH * sizeof(cplx<T>) >= (size_t)ROWS * N * sizeof(double),
-                          "squares of the block's rows fit one exchange buffer");
-            double a = 0.0;
-            if (tid < N) {
+            };
+            if (meth == 3) sums(std::integral_constant<int, 3>{});
+            else sums(std::integral_constant<int, -1>{});
+        };
+        T h[WR];
+        double kk[WR], x2[WR], d2[WR], ah = 0.0, a = 0.0;
 #pragma unroll
-                for (int l = 0; l < LINES; ++l) {
-                    T ha, hb;
-                    dht_pair(xc.at(l, tid), xc.at(l, tid ? N - tid : 0), ha, hb);
-                    const bool inner = l >= 1 && l <= LO;
-                    const bool own = inner && l >= 1 + own0;
-                    const size_t at = (size_t)(2 * gline(l)) * N + tid;
-                    double am = 0.0, da = 0.0, db = 0.0;
-                    cell(2 * l, tid, at, own, ha, xv[2 * l], am, da);
-                    cell(2 * l + 1, tid, at + N, own, hb, xv[2 * l + 1], am, db);
-                    if (inner) {
-                        a = fmax(a, am);
-                        dd[(2 * l - 2) * N + tid] = da;
-                        dd[(2 * l - 1) * N + tid] = db;
+        for (int l = 0; l < LINES; ++l) dht_pair(xc.at(l, col), xc.at(l, col ? N - col : 0), h[2 * l], h[2 * l + 1]);
+        // (the halo rows' maxima are their own blocks')
+        cells(std::integral_constant<int, 2>{}, h, xv, kk, x2, d2, ah);
+        cells(std::integral_constant<int, ROWS>{}, h + 2, xv + 2, kk + 2, x2 + 2, d2 + 2, a);
+        cells(std::integral_constant<int, 2>{}, h + 2 + ROWS, xv + 2 + ROWS, kk + 2 + ROWS, x2 + 2 + ROWS,
+              d2 + 2 + ROWS, ah);
+        if (tid < N) {
+#pragma unroll
+            for (int r = 0; r < WR; ++r) xr[r * N + tid] = x2[r];
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) dd[r * N + tid] = d2[r + 2];
+        }
+        a = wave_max(tid < N ? a : 0.0);
+        if (lane == 0) red[wave] = a;
+        __syncthreads();
+        // the block's own rows to memory
+        if (tid < N) {
+#pragma unroll
+            for (int l = 0; l < LO; ++l)
+                if (l >= own0) {
+                    const size_t at = (size_t)(row0 + 2 * l) * N + tid;
+                    Xn[at] = x2[2 + 2 * l];
+                    Xn[at + N] = x2[3 + 2 * l];
+                    if (ends) {
+                        dw[at] = kk[2 + 2 * l];
+                        dw[at + N] = kk[3 + 2 * l];
                     }
                 }
-            }
-            a = wave_max(a);
-            if (lane == 0) red[wave] = a;
-            __syncthreads();
-            for (int r = wave; r < ROWS; r += NW) {
-                double sm = 0.0;
-                for (int k = lane; k < N; k += 64) sm += dd[r * N + k];
-                sm = wave_sum(sm);
-                // (only the largest maximum of all partials is used: the
-                // block's stands for each of its rows)
-                double am = red[0];
-                for (int w = 1; w < NW; ++w) am = fmax(am, red[w]);
-                if (lane == 0 && r >= 2 * own0) {
-                    gmut<double> pp = part + (size_t)(row0 + r) * 4;
-                    pp[0] = am;
-                    pp[1] = sm;
-                }
-            }
-            __syncthreads();   // the squares' buffer is part of the stencil's
         }
         if (ends) {   // no next attempt if this one is accepted; after a rejection the next kt_turn comes back here
+            partials_sum();
+            __syncthreads();
+            partials_store();
             commit(true);
             return;
         }
@@ -394,8 +426,10 @@ __global__ void __launch_bounds__((Turn<T, N, LO>::THREADS)) kt_turn(const Membe
     }
     __syncthreads();
 
-    // ---- forward row transform of the block's own lines
+    // ---- forward row transform of the block's own lines, the error partials
+    // beside it in the waves that have no line
     {
+        if (!first) partials_sum();
         const bool on = lane_line < LO;
         const int l = on ? lane_line : 0;
         if (on && t < T0) {
@@ -405,6 +439,7 @@ __global__ void __launch_bounds__((Turn<T, N, LO>::THREADS)) kt_turn(const Membe
         }
         MixRow<T, N> xc((cplx<T>*)zreg, LINES, l);
         mix_fft<T, N>(v, t, on, tw_l, xc);
+        if (!first) partials_store();
         gmut<T> dst = gout<T>(M.g2);
         if (tid < N) {
 #pragma unroll
@@ -426,6 +461,7 @@ __global__ void __launch_bounds__((Turn<T, N, LO>::THREADS)) kt_turn(const Membe
 // of a domain transforms copies of its last line where C does not divide N/2.
 template <typename T, int N, int C> struct TurnCol {
     static constexpr int THREADS = (C * MixPlan<N>::TPL + 63) / 64 * 64;
+    // column blocks of a domain, and one more block that only decides
     static constexpr int NB = (N / 2 + C - 1) / C;
     static constexpr size_t lds = ((size_t)N + 2 * (size_t)MixCol<T, N, C>::SIZE) * sizeof(cplx<T>);
 };
@@ -444,6 +480,27 @@ __global__ void __launch_bounds__((TurnCol<T, N, C>::THREADS)) kt_col(const Memb
     const Ctl* const p_ctl = M.ctl;
     const double* const p_part = M.partials;
     scalars_ready(p_src, p_kr, p_ctl, p_part);
+    const kptr<Ctl> c = kview(p_ctl);
+    const kptr<PhysDev> ph = kview(M.phys);
+    if (cblk == TurnCol<T, N, C>::NB) {
+        // the whole decision, to ctl_next, which kt_turn reads and makes
+        // current; the column blocks only find out whether they have to run
+        if ((int)threadIdx.x >= 64) return;
+        StepState st = load_state(c);
+        const bool pending = c->pending != 0;
+        double amax, s2;
+        reduce_partials(gin<double>(p_part), turn_reg8(N) ? N / 2 : N, amax, s2);
+        if (pending) st = decide_step(st, amax, s2, ph, N);
+        if (threadIdx.x == 0) {
+            copy_ctl(M.ctl_next, c);
+            store_state(M.ctl_next, st);
+            M.ctl_next->pending = 0;
+            M.ctl_next->skip = 0;
+        }
+        return;
+    }
+    const int status = c->status, pend = c->pending;
+    const double c_dt = c->dt, c_t = c->t, c_tf = c->tf;
     extern __shared__ __align__(16) unsigned char smem[];
     cplx<T>* tw_l = (cplx<T>*)smem;
     const int tid = threadIdx.x, line = tid % C, t = tid / C;
@@ -452,16 +509,13 @@ __global__ void __launch_bounds__((TurnCol<T, N, C>::THREADS)) kt_col(const Memb
     // the previous attempt's partials first (the decision needs them), then
     // twiddles, spectrum and kappa R; none of them depends on the control block
     constexpr int NP = turn_reg8(N) ? N / 2 : N, PJ = (NP + 63) / 64;
-    double pa[PJ][2];
+    typedef double d2v __attribute__((ext_vector_type(2)));
+    d2v pa[PJ];
     {
-        gptr<double> part = gin<double>(p_part);
+        gptr<d2v> part = gin<d2v>(p_part);
         const int lane = tid & 63;
 #pragma unroll
-        for (int j = 0; j < PJ; ++j) {
-            const int b = lane + 64 * j < NP ? lane + 64 * j : NP - 1;
-#pragma unroll
-            for (int k = 0; k < 2; ++k) pa[j][k] = part[(size_t)b * 4 + k];
-        }
+        for (int j = 0; j < PJ; ++j) pa[j] = part[(size_t)min(lane + 64 * j, NP - 1) * 2];
     }
     constexpr int TWQ = (2 * N + THREADS - 1) / THREADS;
     T twr[TWQ];
@@ -483,47 +537,31 @@ __global__ void __launch_bounds__((TurnCol<T, N, C>::THREADS)) kt_col(const Memb
     for (int r = 0; r < R0; ++r) xk[r] = kR[vec(tt + T0 * r)];
     const double2 wa = tw64[ca], wb = tw64[ca + 1];
     __builtin_amdgcn_sched_barrier(0);
-    const kptr<Ctl> c = kview(p_ctl);
-    StepState st = load_state(c);
-    const bool pending = c->pending != 0;
 #pragma unroll
     for (int k = 0; k < TWQ; ++k)
         if (tid + THREADS * k < 2 * N) ((T*)tw_l)[tid + THREADS * k] = twr[k];
-    // block 0 writes the decided control block to ctl_next, which kt_turn
-    // reads and makes current; every block decides alike
-    auto write_next = [&]() {
-        if (cblk == 0 && tid == 0) {
-            copy_ctl(M.ctl_next, c);
-            store_state(M.ctl_next, st);
-            M.ctl_next->pending = 0;
-            M.ctl_next->skip = 0;
-        }
-    };
-    bool go = st.status == ST_RUN;
-    if (pending) {
+    // Run?  Yes for the first attempt of a round and after an accepted step
+    // that did not end the update; a rejected attempt keeps its right-hand
+    // side, which g1 holds.
+    bool go = status == ST_RUN;
+    if (pend) {
         const int lane = tid & 63;
         double amax = 0.0, s2 = 0.0;
 #pragma unroll
         for (int j = 0; j < PJ; ++j) {
             const bool in = lane + 64 * j < NP;
-            amax = fmax(amax, in ? pa[j][0] : 0.0);
-            s2 += in ? pa[j][1] : 0.0;
+            amax = fmax(amax, in ? pa[j].x : 0.0);
+            s2 += in ? pa[j].y : 0.0;
         }
         amax = wave_max(amax);
         s2 = wave_sum(s2);
-        const long long acc = st.accepts;
-        st = decide_step(st, amax, s2, kview(M.phys), N);
-        // a rejected attempt keeps its right-hand side: g1 holds it
-        go = __builtin_amdgcn_readfirstlane(st.status == ST_RUN && st.accepts != acc);
+        go = __builtin_amdgcn_readfirstlane(step_goes_on(c_dt, c_t, c_tf, amax, s2, ph, N));
     }
-    if (!go) {
-        write_next();
-        return;
-    }
+    if (!go) return;
     cplx<T> v[PL::E];
 #pragma unroll
     for (int r = 0; r < R0; ++r) v[r] = mk<T>(xs[r].x, xs[r].y);
-    __syncthreads();
+    if constexpr (!PL::PLAIN0) __syncthreads();
     MixCol<T, N, C> xc((cplx<T>*)smem + N, line);
     mix_fft<T, N>(v, t, on, tw_l, xc);
     const bool has = on && t < T0;
@@ -553,7 +591,7 @@ __global__ void __launch_bounds__((TurnCol<T, N, C>::THREADS)) kt_col(const Memb
             dst[vec(k)] = o;
             // per-column terms of the four corners of the inverse transform
             // (rows 0 and N-1, weights 1 and cas(2 pi col (N-1) / N))
-            if (k == 0 || k == N - 1) {
+            if ((r == 0 && k == 0) || (r == R0 - 1 && k == N - 1)) {
                 const int q = (k == 0) ? 0 : 2;
                 const double va = (double)ha, vb = (double)hb;
                 cor[(size_t)ca * 4 + q] = va;
@@ -563,7 +601,6 @@ __global__ void __launch_bounds__((TurnCol<T, N, C>::THREADS)) kt_col(const Memb
             }
         }
     }
-    write_next();
 }
 
 // ------------------------------------------------------------------ launchers
@@ -589,7 +626,7 @@ bool turn_cols(const Member* d, int nmem, const RhsShape& s, hipStream_t st, int
     using TC = TurnCol<T, N, C>;
     static const bool ok = turn_lds_ok(kt_col<T, N, C>, TC::lds);
     if (!ok || which < 0) return ok;
-    launch_k(2, kt_col<T, N, C>, dim3(TC::NB, nmem), dim3(TC::THREADS), TC::lds, st, d, s.tw, s.tw64);
+    launch_k(2, kt_col<T, N, C>, dim3(TC::NB + 1, nmem), dim3(TC::THREADS), TC::lds, st, d, s.tw, s.tw64);
     return true;
 }
 

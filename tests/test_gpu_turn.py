@@ -50,7 +50,10 @@ def _run(n, prec, distorted, members):
     (96, "mixed", True, 3), (126, "mixed", False, 1), (128, "mixed", True, 2), (162, "fp64", False, 1),
     (192, "mixed", False, 1), (192, "fp64", True, 1), (200, "mixed", False, 40), (240, "fp64", False, 2),
     (250, "mixed", False, 6), (256, "mixed", False, 1), (256, "fp64", True, 1), (320, "mixed", True, 1),
-    (384, "mixed", False, 1), (486, "mixed", False, 1), (500, "fp64", False, 1), (512, "fp64", False, 1)])
+    (384, "mixed", False, 1), (486, "mixed", False, 1), (500, "fp64", False, 1), (512, "fp64", False, 1),
+    # the register kernels' lengths in blocks of two line pairs, eight columns pairs
+    (64, "fp64", False, 16), (192, "mixed", False, 5), (256, "mixed", False, 4), (384, "fp64", False, 2),
+    (512, "mixed", False, 2)])
 def test_turn_bitwise(n, prec, distorted, members, monkeypatch):
     print(f"case: two-launch attempts N={n} {prec} distorted={distorted} members={members}", flush=True)
     for k in SHAPE_ENV:
