@@ -9,7 +9,8 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libfastiso.so")
-SOURCES = ["rhs_fast.hip"] + ["rhs_turn%d.hip" % k for k in range(8)] + ["rhs.hip", "sealevel.hip", "init.hip", "conv.hip", "kelvin.cpp", "rheogrid.cpp", "api.cpp",
+SOURCES = ["rhs_fast.hip"] + ["rhs_turn%d.hip" % k for k in range(8)] + \
+          ["conv_mix%d.hip" % k for k in range(8)] + ["rhs.hip", "sealevel.hip", "init.hip", "conv.hip", "kelvin.cpp", "rheogrid.cpp", "api.cpp",
            "output.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [

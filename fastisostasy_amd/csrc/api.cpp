@@ -455,6 +455,11 @@ int make_conv_shape(int n, bool fp64, ConvShape& s) {
     s.Lr = L;
     s.Cc = C;
     s.rows_twl = fits(L + 1);
+    // The grouped register passes wherever they exist.  Rows are paired as in
+    // the kernels whose FP32 rounding they keep: neighbours where 2N = 2^k,
+    // l and l + L in blocks of 2L rows elsewhere (FP64: neighbours).
+    s.mix = std::getenv("FI_GENERIC_FFT") ? nullptr : conv_find(n, fp64);
+    s.pair = fp64 || (s.m & (s.m - 1)) == 0 ? 1 : L;
     int rc = fft_threads(s.plan, L, s.threads_row);
     if (rc) return rc;
     rc = fft_threads(s.plan, C, s.threads_col);

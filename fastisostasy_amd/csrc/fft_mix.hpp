@@ -156,6 +156,19 @@ template <typename T, int N, int C> struct MixCol {
     __device__ __forceinline__ void flip() { cur ^= 1; }
 };
 
+// The column exchange in one buffer: a second barrier per exchange for half
+// the LDS, where that lets more blocks share a CU.
+template <typename T, int N, int C> struct MixCol1 {
+    static constexpr int SIZE = (N + N / 8 + 1) * C;
+    cplx<T>* base;
+    int line;
+    __device__ __forceinline__ MixCol1(cplx<T>* b, int l) : base(b), line(l) {}
+    __device__ __forceinline__ int addr(int pos) const { return (pos + (pos >> 3)) * C + line; }
+    __device__ __forceinline__ void put(int pos, cplx<T> v) { base[addr(pos)] = v; }
+    __device__ __forceinline__ cplx<T> get(int pos) const { return base[addr(pos)]; }
+    __device__ __forceinline__ void flip() { __syncthreads(); }
+};
+
 // Forward FFT of the thread's line from group G on.  Entry: v[r] holds element
 // t + (N/R) r of the group's input (threads t < N/R).  Exit: the transform lies
 // in the exchange's current buffer, published by a barrier; the caller reads

@@ -41,6 +41,12 @@ struct RhsShape {
     int turn_LO;      // line pairs per kt_turn block (1 or 2)
 };
 
+// The three passes of a convolution of one length and precision (conv_mix.hpp):
+// (domains, count, twiddles, which, row pairing, stream); false: the device
+// refuses the kernels' LDS
+using ConvFn = bool (*)(const Member*, int, const void*, int, int, hipStream_t);
+ConvFn conv_find(int n, bool fp64);   // null: no such length
+
 // Geometry of the 2N-point linear convolution.
 struct ConvShape {
     int n, m;         // m = 2n
@@ -49,6 +55,8 @@ struct ConvShape {
     FftPlan plan;     // length m
     const void* tw;   // length-m twiddles in conv precision
     bool fp64;
+    ConvFn mix;       // not null: the passes of conv_mix.hpp
+    int pair;         // their row pairing
     bool rows_twl;    // the row passes also hold the twiddle table in LDS (the column pass always does)
 };
 

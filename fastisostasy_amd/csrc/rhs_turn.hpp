@@ -58,6 +58,7 @@ template <typename T, int N, int LO> struct Turn {
     static constexpr size_t zm_bytes = z_bytes > m_bytes ? z_bytes : m_bytes;
     static constexpr size_t lds = tw_bytes + x_bytes + zm_bytes + d_bytes;
     static_assert(N % 2 == 0 && N >= ROWS, "domain smaller than a block");
+    static_assert(THREADS <= 1024, "threads per block");
 };
 
 template <typename T, int N, int LO, bool UNI>
@@ -461,6 +462,7 @@ __global__ void __launch_bounds__((Turn<T, N, LO>::THREADS)) kt_turn(const Membe
 // of a domain transforms copies of its last line where C does not divide N/2.
 template <typename T, int N, int C> struct TurnCol {
     static constexpr int THREADS = (C * MixPlan<N>::TPL + 63) / 64 * 64;
+    static_assert(THREADS <= 1024, "threads per block");
     // column blocks of a domain, and one more block that only decides
     static constexpr int NB = (N / 2 + C - 1) / C;
     static constexpr size_t lds = ((size_t)N + 2 * (size_t)MixCol<T, N, C>::SIZE) * sizeof(cplx<T>);

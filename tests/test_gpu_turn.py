@@ -53,7 +53,9 @@ def _run(n, prec, distorted, members):
     (384, "mixed", False, 1), (486, "mixed", False, 1), (500, "fp64", False, 1), (512, "fp64", False, 1),
     # the register kernels' lengths in blocks of two line pairs, eight columns pairs
     (64, "fp64", False, 16), (192, "mixed", False, 5), (256, "mixed", False, 4), (384, "fp64", False, 2),
-    (512, "mixed", False, 2)])
+    (512, "mixed", False, 2),
+    # the widest column blocks
+    (500, "mixed", False, 2)])
 def test_turn_bitwise(n, prec, distorted, members, monkeypatch):
     print(f"case: two-launch attempts N={n} {prec} distorted={distorted} members={members}", flush=True)
     for k in SHAPE_ENV:
