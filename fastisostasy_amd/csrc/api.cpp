@@ -13,6 +13,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <deque>
 #include <functional>
@@ -501,6 +502,8 @@ struct fi_isos {
     bool use_restart = false;    // a restart was read: the next init_state takes the restart branch
     double time_diag = 0, time_prog = 0;
     double last_t = 0, last_dt = 0;  // ode%t and ode%dt after the last update (host copy; 0 = unknown)
+    double last_span = 0;        // years and attempts of the last update (0: unknown)
+    long long last_attempts = 0, attempts_seen = 0;
     int last_status = 0;         // status of the last update's instability and NaN checks
     char* arena = nullptr;
     size_t arena_bytes = 0;      // HBM footprint of the domain (one allocation)
@@ -582,6 +585,34 @@ void sum_free(SumBuf& b) {
     b.h = nullptr;
 }
 
+// Waiting for the GPU by polling a number that the last kernel of a stream's
+// queued work stores in pinned host memory.  hipStreamSynchronize costs 5 us
+// more on an idle queue and slows the launches after it (ten launches and the
+// wait: 32 us polled, 56 us synchronised).  Work that takes longer than POLL_US
+// is waited for by the runtime, which also reports errors; every 64th wait
+// goes through the runtime too, so that it can retire what it tracks.
+constexpr double POLL_US = 3000.0;
+std::atomic<unsigned> g_wait_seq{0}, g_waits{0};
+unsigned next_seq() { return ++g_wait_seq; }
+
+// done(): whether every awaited number has arrived
+template <class Done> int wait_polled(hipStream_t st, Done&& done) {
+    const auto t0 = std::chrono::steady_clock::now();
+    bool polled = false;
+    for (unsigned k = 0; !(polled = done()); ++k) {
+        __builtin_ia32_pause();
+        if ((k & 63) == 63 &&
+            std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count() > POLL_US)
+            break;
+    }
+    if (polled && (++g_waits & 63) != 0) return 0;
+    HIPCHK(hipStreamSynchronize(st));
+    return done() ? 0 : fail(FI_E_HIP, "the GPU's work ended without its completion number");
+}
+int wait_flag(const unsigned* flag, unsigned v, hipStream_t st) {
+    return wait_polled(st, [=] { return (int)(__atomic_load_n(flag, __ATOMIC_ACQUIRE) - v) >= 0; });
+}
+
 // Pinned host buffers through which fields cross the bus.  A field read back
 // is cropped by a kernel straight into the pinned buffer (one launch and one
 // wait, then a host copy); the ice of an update is copied here and read by the
@@ -595,6 +626,9 @@ struct Stage {
     char* h = nullptr;      // host address
     char* d = nullptr;      // the same memory as the device sees it
     size_t bytes = 0;
+    // completion number, behind the buffer
+    unsigned* flag_h() const { return (unsigned*)(h + bytes); }
+    unsigned* flag_d() const { return (unsigned*)(d + bytes); }
 };
 class StagePool {
     static constexpr size_t UNIT = (size_t)4 << 20, KEEP = (size_t)64 << 20;
@@ -619,7 +653,8 @@ public:
         }
         Stage s;
         s.bytes = (bytes + UNIT - 1) / UNIT * UNIT;
-        HIPCHK(hipHostMalloc((void**)&s.h, s.bytes, hipHostMallocMapped | hipHostMallocCoherent));
+        HIPCHK(hipHostMalloc((void**)&s.h, s.bytes + 64, hipHostMallocMapped | hipHostMallocCoherent));
+        *s.flag_h() = g_wait_seq;
         if (hipHostGetDevicePointer((void**)&s.d, s.h, 0) != hipSuccess) {
             (void)hipHostFree(s.h);
             return fail(FI_E_HIP, "hipHostGetDevicePointer");
@@ -668,13 +703,6 @@ struct StageLease {
         g_stages.give(s);
     }
 };
-
-int gather(Member* d_mem, int nmem, SumBuf& sb) {
-    launch_gather(d_mem, nmem, sb.d, g_stream);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(g_stream));
-    return 0;
-}
 
 // Concurrent sub-batches of the attempt loop (at most three streams besides
 // the library stream, default priority).  One launch of an attempt kernel
@@ -860,6 +888,7 @@ struct UpdateJob {
     bool subbatch = true;        // may split into concurrent sub-batches (library stream only)
     hipStream_t st = nullptr;
     int K = 1, ahead = 1;
+    unsigned seq = 0;            // number of the last round's summaries
     long long total = 0;
     int sb_lo[MAX_SUB + 1] = {};
     const RhsShape* sshape[MAX_SUB] = {};
@@ -892,7 +921,7 @@ int job_begin(UpdateJob& j) {
     if (diag)
         for (fi_isos* h : j.hs) h->time_diag = h->time_diag + h->par.dt_diagnostics;
     launch_pre_haf(d_mem, nmem, n, j.ice, st);
-    launch_pre_bsl(d_mem, nmem, n, st);
+    launch_pre_bsl(d_mem, nmem, n, j.time, j.stepping ? 1 : 0, j.times != nullptr, st);
     if (!diag) {
         launch_pre_fields(d_mem, nmem, n, 0, false, h0.fp64, st);
     } else if (!h0.par.include_elastic && !h0.par.heterogeneous_ssh) {
@@ -908,7 +937,6 @@ int job_begin(UpdateJob& j) {
             launch_pre_fields(d_mem, nmem, n, 4, true, h0.fp64, st);   // phases 1-2 in one pass
         }
     }
-    launch_begin(d_mem, nmem, j.time, j.stepping ? 1 : 0, j.times != nullptr, st);
     if (j.stepping && shape.method != 3) {
         if (shape.method == 2) {
             launch_weq_input(d_mem, nmem, n, st);
@@ -923,10 +951,19 @@ int job_begin(UpdateJob& j) {
     // round launches as many attempts as the slowest member needs at the dt it
     // ended its previous update with, plus a margin for rejections; after each
     // readback job_more corrects the estimate.
-    double need = 0.0;
-    for (int m = 0; m < nmem; ++m)
-        if (j.hs[m]->last_dt > 0.0) need = std::max(need, std::ceil((j.t_of(m) - j.hs[m]->last_t) / j.hs[m]->last_dt));
+    // A load that changes from one coupling step to the next cuts the step at
+    // the start of each update: then the last update of the same span is the
+    // better guess (N = 64 disc under varying ice: 6-7 attempts where the last dt
+    // promises one; a second round costs about 25 us, an unused attempt 4).
+    double need = 0.0, again = 0.0;
+    for (int m = 0; m < nmem; ++m) {
+        const fi_isos& h = *j.hs[m];
+        const double span = j.t_of(m) - h.last_t;
+        if (h.last_dt > 0.0) need = std::max(need, std::ceil(span / h.last_dt));
+        if (std::fabs(span - h.last_span) <= 1e-6 * span) again = std::max(again, (double)h.last_attempts);
+    }
     if (need > 0.0) need += (double)first_round_margin();
+    if (again > need) need = again + 1.0;
     j.ahead = (int)std::min(256.0, std::max(1.0, need));
     // concurrent sub-batches only on the library stream (their streams are shared)
     j.K = shape.method == 3 && j.st == g_stream && j.subbatch ? sub_count(n, h0.fp64, nmem) : 1;
@@ -956,7 +993,7 @@ int job_round(UpdateJob& j) {
             launch_round_start(d_mem, nmem, shape, j.st);
             int rc = launch_attempts(d_mem, nmem, shape, j.st, j.ahead, j.graphs);
             if (rc) return rc;
-            launch_decide(d_mem, nmem, shape, j.st);
+            launch_round_end(d_mem, nmem, shape, j.st);
         } else {
             HIPCHK(hipEventRecord(g_sub.start, j.st));
             for (int k = 0; k < j.K; ++k) HIPCHK(hipStreamWaitEvent(g_sub.s[k], g_sub.start, 0));
@@ -970,16 +1007,17 @@ int job_round(UpdateJob& j) {
                     if (rc) return rc;
                 }
             for (int k = 0; k < j.K; ++k) {
-                launch_decide(d_mem + j.sb_lo[k], j.sb_lo[k + 1] - j.sb_lo[k], *j.sshape[k], g_sub.s[k]);
+                launch_round_end(d_mem + j.sb_lo[k], j.sb_lo[k + 1] - j.sb_lo[k], *j.sshape[k], g_sub.s[k]);
                 HIPCHK(hipEventRecord(g_sub.done[k], g_sub.s[k]));
                 HIPCHK(hipStreamWaitEvent(j.st, g_sub.done[k], 0));
             }
         }
         j.total += j.ahead;
+    } else {
+        launch_round_end(d_mem, nmem, shape, j.st);
     }
-    launch_finalize(d_mem, nmem, n, j.st);
-    HIPCHK(hipGetLastError());
-    launch_gather(d_mem, nmem, j.sb.d, j.st);   // stores into pinned host memory
+    j.seq = next_seq();
+    launch_finalize(d_mem, nmem, n, j.sb.d, j.seq, j.st);   // stores the summaries into pinned host memory
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -1032,6 +1070,9 @@ int job_end(UpdateJob& j) {
         const CtlSummary& c = j.sb.h[m];
         fi_isos* h = j.hs[m];
         h->time_prog = j.t_of(m);
+        h->last_span = j.stepping && h->last_dt > 0.0 ? c.t - h->last_t : 0.0;
+        h->last_attempts = c.attempts - h->attempts_seen;
+        h->attempts_seen = c.attempts;
         h->last_t = c.t;
         h->last_dt = j.stepping ? c.dt : 0.0;
         const char* what;
@@ -1062,7 +1103,12 @@ int run_update(std::vector<fi_isos*>& hs, Member* d_mem, const RhsShape& shape, 
     for (;;) {
         rc = job_round(j);
         if (rc) return rc;
-        HIPCHK(hipStreamSynchronize(j.st));
+        rc = wait_polled(j.st, [&] {
+            for (size_t m = 0; m < j.hs.size(); ++m)
+                if (__atomic_load_n(&j.sb.h[m].seq, __ATOMIC_ACQUIRE) != j.seq) return false;
+            return true;
+        });
+        if (rc) return rc;
         bool more = false;
         rc = job_more(j, more);
         if (rc) return rc;
@@ -1094,28 +1140,18 @@ int read_window(fi_isos* h, const void* src, int bit, int i0, int j0, int ni, in
     StageLease st;
     int rc = st.take(sizeof(T) * ni * nj);
     if (rc) return rc;
-    // the events of the chunks before the last (the last one's end is the stream's)
-    struct Events {
-        std::vector<hipEvent_t> e;
-        ~Events() {
-            for (hipEvent_t x : e) (void)hipEventDestroy(x);
-        }
-    } ev;
+    // (numbers rise from chunk to chunk; another thread's may lie between)
+    std::vector<unsigned> seq(nch);
     for (int c = 0; c < nch; ++c) {
         const int j = c * rows, nr = std::min(rows, nj - j);
         launch_crop(src, bit, h->n, i0, j0 + j, ni, nr, st.s.d + sizeof(T) * (size_t)j * ni, g_stream);
+        launch_flag(st.s.flag_d(), seq[c] = next_seq(), g_stream);
         HIPCHK(hipGetLastError());
-        if (c + 1 < nch) {
-            hipEvent_t e = nullptr;
-            HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-            ev.e.push_back(e);
-            HIPCHK(hipEventRecord(e, g_stream));
-        }
     }
     for (int c = 0; c < nch; ++c) {
         const int j = c * rows, nr = std::min(rows, nj - j);
-        if (c + 1 < nch) HIPCHK(hipEventSynchronize(ev.e[c]));
-        else HIPCHK(hipStreamSynchronize(g_stream));
+        rc = wait_flag(st.s.flag_h(), seq[c], g_stream);
+        if (rc) return rc;
         const size_t at = (size_t)j * ni;
         put(at, (size_t)nr * ni, (const T*)st.s.h + at);
     }
@@ -1664,6 +1700,10 @@ int fi_isos_init_state(fi_isos* h, const double* z_bed, const double* H_ice, dou
     c.k_valid = 0;
     rc = write_ctl(M, c);
     if (rc) return rc;
+    // (the first update's launch estimate starts from dt_init)
+    h->last_t = time;
+    h->last_dt = h->par.dt_init;
+    h->last_span = 0.0;
     h->state_init = true;
     h->use_restart = false;
     return 0;

@@ -63,8 +63,10 @@ struct ConvShape {
 // before the first attempt of a launch round (two-launch attempts only)
 void launch_round_start(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st);
 void launch_attempt(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st);
-// applies a pending step decision left by the last attempt (no-op otherwise)
-void launch_decide(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st);
+// the end of a launch round: applies a pending step decision left by the last
+// attempt and, for domains that have stopped stepping, forms the corner
+// correction of now%w (launch_finalize follows)
+void launch_round_end(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st);
 // power-of-two passes: which = 1 row forward, 2 column, 3 row inverse
 bool launch_fast_pass(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st, int which);
 // LDS exchange buffers (1 or 2) of the column pass launched for shape s
@@ -104,14 +106,15 @@ void launch_pre_haf(const Member* d_mem, int nmem, int n, const double* ice, hip
 // rows [j0, j0 + nj) x columns [i0, i0 + ni) of an n x n field into dst (contiguous
 // doubles), or, with bit != 0, of that bit of an n x n byte mask (contiguous bytes 0 / 1)
 void launch_crop(const void* src, int bit, int n, int i0, int j0, int ni, int nj, void* dst, hipStream_t st);
-void launch_pre_bsl(const Member* d_mem, int nmem, int n, hipStream_t st);
+void launch_pre_bsl(const Member* d_mem, int nmem, int n, double tf, int stepping, bool per_member, hipStream_t st);
 // phase 0: z_ss/masks/loads and, without diagnostics, everything the RHS needs
 // phase 1: (after the elastic convolution) litho/full/mass anomaly
 // phase 2: (after the sea-surface convolution) z_ss/masks/loads/full
 void launch_pre_fields(const Member* d_mem, int nmem, int n, int phase, bool diag, bool fp64, hipStream_t st);
-void launch_begin(const Member* d_mem, int nmem, double tf, int stepping, bool per_member, hipStream_t st);
-void launch_finalize(const Member* d_mem, int nmem, int n, hipStream_t st);
-void launch_gather(const Member* d_mem, int nmem, CtlSummary* d_out, hipStream_t st);
+// finalizes the domains that are done and stores every domain's summary, numbered seq
+void launch_finalize(const Member* d_mem, int nmem, int n, CtlSummary* d_out, unsigned seq, hipStream_t st);
+// *flag (pinned host memory) = v once all work queued before has ended
+void launch_flag(unsigned* flag, unsigned v, hipStream_t st);
 void launch_bsl_update(BslDev* b, double year_bp, double file_value, hipStream_t st);
 // methods 0-2: w_equilibrium of the update (lv_xlra.f90, fastisostasy.f90:686-714);
 // method 2 first stages -canom_load g K^2 (launch_weq_input), then convolves it

@@ -44,10 +44,13 @@ struct Ctl {
 // ST_NAN: stepping stopped by a NaN error norm (reported as FI_E_NAN)
 enum { ST_IDLE = 0, ST_RUN = 1, ST_NAN = -1 };
 
-// Host-visible summary of one domain, gathered after a group of launches.
+// Host-visible summary of one domain, stored at the end of a launch round.
 struct CtlSummary {
     double t, dt, tf, maxw, maxwe, maxdzss, maxweq;
+    long long attempts;
     int status, nonfinite;
+    unsigned seq;                // round that stored it, written last
+    int pad_;
 };
 
 // Barystatic sea level, resident in device memory (bsl_class,

@@ -433,6 +433,28 @@ __global__ void __launch_bounds__(64) k_decide(const Member* __restrict__ mem, i
     decide_wave(mem[blockIdx.x], nblk);
 }
 
+// The end of a launch round, one wave per domain: the decision of the last
+// attempt, and the corner correction of now%w (isos_utils.f90:104-110) of a
+// domain that has stopped stepping and is not finalized yet.
+__global__ void __launch_bounds__(64) k_round_end(const Member* __restrict__ mem, int nblk) {
+    const Member& M = mem[blockIdx.x];
+    const kptr<Ctl> ck = kview(M.ctl);
+    StepState s = load_state(ck);
+    const int pending = ck->pending, fin = ck->fin;
+    double amax, s2;
+    reduce_partials(gin<double>(M.partials), nblk, amax, s2);
+    if (threadIdx.x != 0) return;
+    if (pending) {
+        s = decide_step(s, amax, s2, kview(M.phys), M.n);
+        store_state(M.ctl, s);
+        M.ctl->pending = 0;
+    }
+    if (s.status == ST_RUN || fin) return;
+    const int N = M.n;
+    const double* w = s.w_is_x ? M.X[s.cur] : M.W;
+    M.ctl->wcorner = 0.25 * (w[0] + w[(size_t)N * N - 1] + w[(size_t)(N - 1) * N] + w[N - 1]);
+}
+
 // ------------------------------------------------------------------ launchers
 template <typename T>
 static size_t lds_bytes(int n, int lines) { return (size_t)n * (lines + 1) * sizeof(cplx<T>); }   // + twiddles
@@ -553,14 +575,14 @@ void launch_attempt_t(const Member* d_mem, int nmem, const RhsShape& s, hipStrea
         nblk = s.n;
     }
     // the fused pass of the next attempt applies this attempt's decision; the
-    // last one of a launch round is applied by launch_decide
+    // last one of a launch round is applied by launch_round_end
     if (!fused) hipLaunchKernelGGL(k_decide, dim3(nmem), dim3(64), 0, st, d_mem, nblk);
 }
 
-void launch_decide(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st) {
+void launch_round_end(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st) {
     // partials: one per line pair of rows on the register kernels, one per row on the mixed-radix LDS kernels
     const int nblk = s.fast ? s.n / 2 : s.n;
-    hipLaunchKernelGGL(k_decide, dim3(nmem), dim3(64), 0, st, d_mem, nblk);
+    hipLaunchKernelGGL(k_round_end, dim3(nmem), dim3(64), 0, st, d_mem, nblk);
 }
 
 void launch_attempt(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st) {

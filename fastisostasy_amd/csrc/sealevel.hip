@@ -119,7 +119,10 @@ __global__ void __launch_bounds__(PRE_THREADS) k_pre_haf(const Member* __restric
     }
 }
 
-__global__ void __launch_bounds__(64) k_pre_bsl(const Member* __restrict__ mem, int nmem, int nblk) {
+// Also begins the update: the target time (tf, or the domain's own tf_req) and
+// the stepping flags, so that no launch of its own is needed for them.
+__global__ void __launch_bounds__(64) k_pre_bsl(const Member* __restrict__ mem, int nmem, int nblk, double tf,
+                                                int stepping, int per_member) {
     const int lane = threadIdx.x;
     if (!mem[blockIdx.x].bsl_lead) return;
     for (int m = blockIdx.x; m >= 0 && m < nmem; m = mem[m].bsl_next) {
@@ -143,6 +146,13 @@ __global__ void __launch_bounds__(64) k_pre_bsl(const Member* __restrict__ mem, 
                 b.bsl_now = b.bsl_now - c.dbsl_total;
             }
             c.bsl = b.bsl_now;
+            const double target = per_member ? M.tf_req : tf;
+            c.tf = target;
+            c.k_valid = 0;
+            c.pending = 0;
+            c.skip = 0;
+            c.fin = 0;
+            c.status = (stepping && c.t < target) ? ST_RUN : ST_IDLE;
         }
         __syncthreads();
     }
@@ -328,21 +338,10 @@ void launch_weq(const Member* d_mem, int nmem, int n, int method, hipStream_t st
     hipLaunchKernelGGL(k_weq, dim3(nmem), dim3(WEQ_THREADS), 0, st, d_mem, method);
 }
 
-// Corner correction of now%w (isos_utils.f90:104-110), one thread per domain.
 // The finalize kernels run once per update and domain, for domains that have
-// stopped stepping: the host may launch them before it knows that every
-// domain is done, and again after further attempts.
-__global__ void k_fin_corner(const Member* __restrict__ mem, int nmem) {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= nmem) return;
-    const Member& M = mem[m];
-    Ctl& c = *M.ctl;
-    if (c.status == ST_RUN || c.fin) return;
-    const int N = M.n;
-    const double* w = c.w_is_x ? M.X[c.cur] : M.W;
-    c.wcorner = 0.25 * (w[0] + w[(size_t)N * N - 1] + w[(size_t)(N - 1) * N] + w[N - 1]);
-}
-
+// stopped stepping (k_round_end in rhs.hip left their corner correction of
+// now%w): the host may launch them before it knows that every domain is done,
+// and again after further attempts.
 __global__ void __launch_bounds__(PRE_THREADS) k_finalize(const Member* __restrict__ mem) {
     const Member& M = mem[blockIdx.y];
     const kptr<PhysDev> ph = kview(M.phys);
@@ -399,48 +398,33 @@ __global__ void __launch_bounds__(PRE_THREADS) k_finalize(const Member* __restri
     }
 }
 
-__global__ void __launch_bounds__(64) k_fin_check(const Member* __restrict__ mem, int nblk) {
+// The checks of a finalized domain, and every domain's summary to the host.
+__global__ void __launch_bounds__(64) k_fin_check(const Member* __restrict__ mem, int nblk,
+                                                  CtlSummary* __restrict__ out, unsigned seq) {
     const Member& M = mem[blockIdx.x];
     Ctl& c = *M.ctl;
-    if (c.status == ST_RUN || c.fin) return;
-    double v[FIN_P] = {0, 0, 0, 0, 0};
-    for (int b = threadIdx.x; b < nblk; b += 64)
-        for (int r = 0; r < FIN_P; ++r) v[r] = fmax(v[r], M.partials[(size_t)b * FIN_P + r]);
-    for (int r = 0; r < FIN_P; ++r) v[r] = wave_max(v[r]);
-    if (threadIdx.x == 0) {
-        c.maxw = v[0]; c.maxwe = v[1]; c.maxdzss = v[2]; c.maxweq = v[4];
-        c.nonfinite = v[3] > 0.0 || c.status == ST_NAN;
-        c.w_is_x = 0;
-        c.status = ST_IDLE;
-        c.fin = 1;
+    if (c.status != ST_RUN && !c.fin) {
+        double v[FIN_P] = {0, 0, 0, 0, 0};
+        for (int b = threadIdx.x; b < nblk; b += 64)
+            for (int r = 0; r < FIN_P; ++r) v[r] = fmax(v[r], M.partials[(size_t)b * FIN_P + r]);
+        for (int r = 0; r < FIN_P; ++r) v[r] = wave_max(v[r]);
+        if (threadIdx.x == 0) {
+            c.maxw = v[0]; c.maxwe = v[1]; c.maxdzss = v[2]; c.maxweq = v[4];
+            c.nonfinite = v[3] > 0.0 || c.status == ST_NAN;
+            c.w_is_x = 0;
+            c.status = ST_IDLE;
+            c.fin = 1;
+        }
     }
-}
-
-__global__ void k_begin(const Member* __restrict__ mem, int nmem, double tf, int stepping, int per_member) {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= nmem) return;
-    Ctl& c = *mem[m].ctl;
-    if (per_member) tf = mem[m].tf_req;
-    c.tf = tf;
-    c.k_valid = 0;
-    c.pending = 0;
-    c.skip = 0;
-    c.fin = 0;
-    c.status = (stepping && c.t < tf) ? ST_RUN : ST_IDLE;
-}
-
-__global__ void k_gather(const Member* __restrict__ mem, int nmem, CtlSummary* __restrict__ out) {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= nmem) return;
-    const Ctl& c = *mem[m].ctl;
-    CtlSummary s;
-    s.t = c.t; s.dt = c.dt; s.tf = c.tf; s.maxw = c.maxw; s.maxwe = c.maxwe; s.maxdzss = c.maxdzss; s.maxweq = c.maxweq;
-    s.status = c.status; s.nonfinite = c.nonfinite;
-    out[m] = s;
-}
-
-void launch_gather(const Member* d_mem, int nmem, CtlSummary* d_out, hipStream_t st) {
-    hipLaunchKernelGGL(k_gather, dim3((nmem + 63) / 64), dim3(64), 0, st, d_mem, nmem, d_out);
+    if (threadIdx.x == 0) {
+        CtlSummary& s = out[blockIdx.x];
+        s.t = c.t; s.dt = c.dt; s.tf = c.tf; s.maxw = c.maxw; s.maxwe = c.maxwe; s.maxdzss = c.maxdzss;
+        s.maxweq = c.maxweq;
+        s.attempts = c.attempts;
+        s.status = c.status; s.nonfinite = c.nonfinite;
+        // the host polls the round's number
+        __hip_atomic_store(&s.seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // barysealevel.f90:195-252 (const / fastiso / file / mixed), one thread
@@ -518,6 +502,14 @@ __global__ void __launch_bounds__(256) k_crop_mask(const uint8_t* __restrict__ s
     if (q >= count) return;
     dst[q] = (src[(size_t)(j0 + q / ni) * n + i0 + q % ni] & bit) ? 1 : 0;
 }
+// Tells the polling host that everything queued before it has ended: the
+// windows' stores are complete at the end of their kernel.
+__global__ void k_flag(unsigned* flag, unsigned v) {
+    __hip_atomic_store(flag, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+void launch_flag(unsigned* flag, unsigned v, hipStream_t st) {
+    hipLaunchKernelGGL(k_flag, dim3(1), dim3(1), 0, st, flag, v);
+}
 void launch_crop(const void* src, int bit, int n, int i0, int j0, int ni, int nj, void* dst, hipStream_t st) {
     const int count = ni * nj;
     const dim3 g((count + 255) / 256), b(256);
@@ -526,8 +518,9 @@ void launch_crop(const void* src, int bit, int n, int i0, int j0, int ni, int nj
     else
         hipLaunchKernelGGL(k_crop, g, b, 0, st, (const double*)src, n, i0, j0, ni, count, (double*)dst);
 }
-void launch_pre_bsl(const Member* d_mem, int nmem, int n, hipStream_t st) {
-    hipLaunchKernelGGL(k_pre_bsl, dim3(nmem), dim3(64), 0, st, d_mem, nmem, pre_blocks(n));
+void launch_pre_bsl(const Member* d_mem, int nmem, int n, double tf, int stepping, bool per_member, hipStream_t st) {
+    hipLaunchKernelGGL(k_pre_bsl, dim3(nmem), dim3(64), 0, st, d_mem, nmem, pre_blocks(n), tf, stepping,
+                       per_member ? 1 : 0);
 }
 template <typename T>
 static void pre_fields_t(const Member* d_mem, int nmem, int n, int phase, bool diag, hipStream_t st) {
@@ -548,14 +541,9 @@ void launch_pre_fields(const Member* d_mem, int nmem, int n, int phase, bool dia
     if (fp64) pre_fields_t<double>(d_mem, nmem, n, phase, diag, st);
     else pre_fields_t<float>(d_mem, nmem, n, phase, diag, st);
 }
-void launch_begin(const Member* d_mem, int nmem, double tf, int stepping, bool per_member, hipStream_t st) {
-    hipLaunchKernelGGL(k_begin, dim3((nmem + 63) / 64), dim3(64), 0, st, d_mem, nmem, tf, stepping,
-                       per_member ? 1 : 0);
-}
-void launch_finalize(const Member* d_mem, int nmem, int n, hipStream_t st) {
-    hipLaunchKernelGGL(k_fin_corner, dim3((nmem + 63) / 64), dim3(64), 0, st, d_mem, nmem);
+void launch_finalize(const Member* d_mem, int nmem, int n, CtlSummary* d_out, unsigned seq, hipStream_t st) {
     hipLaunchKernelGGL(k_finalize, dim3(pre_blocks(n), nmem), dim3(PRE_THREADS), 0, st, d_mem);
-    hipLaunchKernelGGL(k_fin_check, dim3(nmem), dim3(64), 0, st, d_mem, pre_blocks(n));
+    hipLaunchKernelGGL(k_fin_check, dim3(nmem), dim3(64), 0, st, d_mem, pre_blocks(n), d_out, seq);
 }
 void launch_bsl_update(BslDev* b, double year_bp, double file_value, hipStream_t st) {
     hipLaunchKernelGGL(k_bsl_update, dim3(1), dim3(1), 0, st, b, year_bp, file_value);
