@@ -815,7 +815,7 @@ int attempt_graph(const Member* d, int nmem, const RhsShape& s, hipStream_t st, 
             return 0;
         }
     HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    for (int r = 0; r < GRAPH_REPS; ++r) launch_attempt(d, nmem, s, st);
+    for (int r = 0; r < GRAPH_REPS; r += attempts_per_launch(s)) launch_attempt(d, nmem, s, st);
     hipGraph_t g = nullptr;
     HIPCHK(hipStreamEndCapture(st, &g));
     hipGraphExec_t ex = nullptr;
@@ -859,7 +859,8 @@ int launch_attempts(const Member* d, int nmem, const RhsShape& s, hipStream_t st
         if (rc) return rc;
         for (; done + GRAPH_REPS <= count; done += GRAPH_REPS) HIPCHK(hipGraphLaunch(ex, st));
     }
-    for (; done < count; ++done) launch_attempt(d, nmem, s, st);
+    const int per = attempts_per_launch(s);
+    for (; done < count; done += per) launch_attempt(d, nmem, s, st);
     return 0;
 }
 
@@ -1315,6 +1316,11 @@ int fi_bsl_update(fi_bsl* b, double year_bp) {
     // bsl_update_file (barysealevel.f90:230-238): the series at the caller's time
     const double file_value =
         b->st.empty() ? 0.0 : interp_first_ge(b->st.data(), b->sv.data(), (int)b->st.size(), year_bp);
+    // Nothing on the device changes for the methods const, and fastiso with a
+    // constant ocean surface (their A_ocean and bsl_init are set at create; the
+    // time is only kept): no launch, 3.4 us of host and 2 of GPU time per object.
+    b->h.time = year_bp;
+    if (b->h.method == 0 || (b->h.method == 1 && b->h.constant_ocean_surface)) return 0;
     launch_bsl_update(b->d, year_bp, file_value, g_stream);
     HIPCHK(hipGetLastError());
     return 0;
@@ -1322,8 +1328,10 @@ int fi_bsl_update(fi_bsl* b, double year_bp) {
 
 int fi_bsl_get(fi_bsl* b, double* bsl_now, double* A_ocean_now) {
     if (!b) return fail(FI_E_ARG, "bsl is NULL");
+    const double year = b->h.time;
     HIPCHK(hipMemcpyAsync(&b->h, b->d, sizeof(BslDev), hipMemcpyDeviceToHost, g_stream));
     HIPCHK(hipStreamSynchronize(g_stream));
+    b->h.time = year;
     if (bsl_now) *bsl_now = b->h.bsl_now;
     if (A_ocean_now) *A_ocean_now = b->h.A_ocean_now;
     return 0;

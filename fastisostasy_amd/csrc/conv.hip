@@ -155,7 +155,8 @@ __global__ void __launch_bounds__(512) c_rows_c2r(const Member* __restrict__ mem
     const double scale = (double)Mm * (double)Mm;
     const double cc = corr;
     const int c0 = N / 2 - 1 + (N % 2);
-    double* out = (which == 0) ? M.we : (which == 1) ? M.dz_ss : M.weq;
+    // (the viscous convolution goes to the state buffer that is free until the first attempt, k_weq)
+    double* out = (which == 0) ? M.we : (which == 1) ? M.dz_ss : M.X[M.ctl->cur ^ 1];
     for (int q = tid; q < 2 * L * N; q += nt) {
         const int mr = q / N, i = q % N;
         const int l = mr % L, part = mr / L;

@@ -199,7 +199,8 @@ __global__ void __launch_bounds__((ConvMix<T, M>::TR)) cm_rows_c2r(const Member*
     MixRow<T, M> xc(tw_l + M, LB, line < LB ? line : 0);
     mix_fft<T, M>(v, t, on, tw_l, xc);
     const double scale = (double)M * (double)M;
-    gmut<double> out = gout<double>((which == 0) ? Mb.we : (which == 1) ? Mb.dz_ss : Mb.weq);
+    // (the viscous convolution goes to the state buffer that is free until the first attempt, k_weq)
+    gmut<double> out = gout<double>((which == 0) ? Mb.we : (which == 1) ? Mb.dz_ss : Mb.X[Mb.ctl->cur ^ 1]);
     for (int q = tid; q < LB * N; q += CM::TR) {
         const int l = q / N, i = q - l * N;
         if (j0 + l >= N / 2) break;

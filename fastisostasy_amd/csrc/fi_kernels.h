@@ -62,6 +62,8 @@ struct ConvShape {
 
 // before the first attempt of a launch round (two-launch attempts only)
 void launch_round_start(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st);
+// one attempt; two for methods 0-2 (attempts_per_launch)
+inline int attempts_per_launch(const RhsShape& s) { return s.method != 3 ? 2 : 1; }
 void launch_attempt(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st);
 // the end of a launch round: applies a pending step decision left by the last
 // attempt and, for domains that have stopped stepping, forms the corner

@@ -397,21 +397,46 @@ __global__ void __launch_bounds__(512) k_row_inv(const Member* __restrict__ mem,
 // (calc_asthenosphere_relax, lv_xlra.f90:17-26; 0 for method 0), stage sums
 // and error partials.  One block per pair of rows, so the partials have the
 // layout of the power-of-two LV-ELVA path (one entry per row pair).
+//
+// One launch per attempt: every wave first applies the previous attempt's
+// decision from its partials.  Attempts of a round alternate between two
+// control blocks and two sets of partials (parity p reads ctl[p] and set
+// 1 - p, block 0 writes ctl[1 - p], everyone writes set p), so nothing is
+// written that another block still reads; a round runs an even number of
+// attempts and ends in M.ctl and set 1.  (N = 256: 4.9 us per attempt against
+// 4.2 + 2.6 with a decision of its own.)
 constexpr int XLRA_THREADS = 256;
-__global__ void __launch_bounds__(XLRA_THREADS) k_xlra(const Member* __restrict__ mem) {
+__device__ __host__ inline size_t xlra_set(int n, int p) { return (size_t)2 * n * p; }   // doubles
+__global__ void __launch_bounds__(XLRA_THREADS) k_xlra(const Member* __restrict__ mem, int p) {
     const Member& M = mem[blockIdx.y];
-    const Ctl& c = *M.ctl;
-    if (c.status != ST_RUN) return;
-    const PhysDev& ph = *M.phys;
+    const kptr<Ctl> c = kview(p ? M.ctl_next : M.ctl);
+    Ctl* const next = p ? M.ctl : M.ctl_next;
+    const kptr<PhysDev> ph = kview(M.phys);
     const int N = M.n;
-    const double dt = attempt_dt(c, ph);
-    const double* __restrict__ X = M.X[c.cur];
-    double* __restrict__ Xn = M.X[c.cur ^ 1];
-    const double* __restrict__ w = c.w_is_x ? X : M.W;
+    StepState st = load_state(c);
+    if (c->pending) {
+        double amax, s2;
+        reduce_partials(gin<double>(M.partials) + xlra_set(N, 1 - p), (N + 1) / 2, amax, s2);
+        st = decide_step(st, amax, s2, ph, N);
+        st.cur = __builtin_amdgcn_readfirstlane(st.cur);
+        st.w_is_x = __builtin_amdgcn_readfirstlane(st.w_is_x);
+        st.status = __builtin_amdgcn_readfirstlane(st.status);
+    }
+    const bool run = st.status == ST_RUN;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        copy_ctl(next, c);
+        store_state(next, st);
+        next->pending = run ? 1 : 0;
+    }
+    if (!run) return;
+    const double dt = attempt_dt(ph->dt_method, st.dt, st.t, st.tf, ph->dt_max);
+    const double* __restrict__ X = M.X[st.cur];
+    double* __restrict__ Xn = M.X[st.cur ^ 1];
+    const double* __restrict__ w = st.w_is_x ? X : M.W;
     const double* __restrict__ weq = M.weq;
-    const bool relax = ph.method != 0, store_k = !(c.t + dt < c.tf);
-    const double tau = ph.tau;
-    const int dtm = ph.dt_method;
+    const bool relax = ph->method != 0, store_k = !(st.t + dt < st.tf);
+    const double tau = ph->tau;
+    const int dtm = ph->dt_method;
     const int r0 = blockIdx.x * 2, rows = min(2, N - r0);
     double a1 = 0.0, a2 = 0.0, s2 = 0.0;
     for (int q = threadIdx.x; q < rows * N; q += XLRA_THREADS) {
@@ -425,8 +450,7 @@ __global__ void __launch_bounds__(XLRA_THREADS) k_xlra(const Member* __restrict_
         const double d = x2 - x1;
         s2 += d * d;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) M.ctl->pending = 1;
-    block_reduce3(a1, a2, s2, M.partials + (size_t)blockIdx.x * 4);
+    block_reduce3(a1, a2, s2, M.partials + xlra_set(N, p) + (size_t)blockIdx.x * 4);
 }
 
 __global__ void __launch_bounds__(64) k_decide(const Member* __restrict__ mem, int nblk) {
@@ -436,13 +460,13 @@ __global__ void __launch_bounds__(64) k_decide(const Member* __restrict__ mem, i
 // The end of a launch round, one wave per domain: the decision of the last
 // attempt, and the corner correction of now%w (isos_utils.f90:104-110) of a
 // domain that has stopped stepping and is not finalized yet.
-__global__ void __launch_bounds__(64) k_round_end(const Member* __restrict__ mem, int nblk) {
+__global__ void __launch_bounds__(64) k_round_end(const Member* __restrict__ mem, int nblk, int xlra) {
     const Member& M = mem[blockIdx.x];
     const kptr<Ctl> ck = kview(M.ctl);
     StepState s = load_state(ck);
     const int pending = ck->pending, fin = ck->fin;
     double amax, s2;
-    reduce_partials(gin<double>(M.partials), nblk, amax, s2);
+    reduce_partials(gin<double>(M.partials) + (xlra ? xlra_set(M.n, 1) : 0), nblk, amax, s2);
     if (threadIdx.x != 0) return;
     if (pending) {
         s = decide_step(s, amax, s2, kview(M.phys), M.n);
@@ -521,11 +545,10 @@ int prof_collect_kernel(int kernel, double* total_ms, long long* launches) {
 
 int prof_collect(double* total_ms, long long* launches) { return prof_collect_kernel(-1, total_ms, launches); }
 
-// methods 0-2: one pointwise kernel, decided at once
+// methods 0-2: two attempts (of parities 0 and 1) of one pointwise kernel each
 void launch_attempt_xlra(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st) {
     const int nblk = (s.n + 1) / 2;
-    launch_k(3, k_xlra, dim3(nblk, nmem), dim3(XLRA_THREADS), 0, st, d_mem);
-    hipLaunchKernelGGL(k_decide, dim3(nmem), dim3(64), 0, st, d_mem, nblk);
+    for (int p = 0; p < 2; ++p) launch_k(3, k_xlra, dim3(nblk, nmem), dim3(XLRA_THREADS), 0, st, d_mem, p);
 }
 
 // two-launch attempts: lengths by translation unit
@@ -580,9 +603,11 @@ void launch_attempt_t(const Member* d_mem, int nmem, const RhsShape& s, hipStrea
 }
 
 void launch_round_end(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st) {
-    // partials: one per line pair of rows on the register kernels, one per row on the mixed-radix LDS kernels
-    const int nblk = s.fast ? s.n / 2 : s.n;
-    hipLaunchKernelGGL(k_round_end, dim3(nmem), dim3(64), 0, st, d_mem, nblk);
+    // partials: one per line pair of rows on the register kernels and for
+    // methods 0-2, one per row on the mixed-radix LDS kernels
+    const bool xlra = s.method != 3;
+    const int nblk = xlra ? (s.n + 1) / 2 : s.fast ? s.n / 2 : s.n;
+    hipLaunchKernelGGL(k_round_end, dim3(nmem), dim3(64), 0, st, d_mem, nblk, xlra ? 1 : 0);
 }
 
 void launch_attempt(const Member* d_mem, int nmem, const RhsShape& s, hipStream_t st) {

@@ -302,29 +302,27 @@ __global__ void __launch_bounds__(PRE_THREADS) k_weq_input(const Member* __restr
 // reference recomputes it in every RHS call from fields that stay fixed
 // during the update: get_dwdt, fastisostasy.f90:686-714).
 //   0: 0;  1: -canom_load / rho_uppermantle (lv_xlra.f90:29-38);
-//   2: corner BC (isos_utils.f90:104-118) of the viscous convolution in weq.
-// One block per domain, so the corner values are read before any is changed.
-constexpr int WEQ_THREADS = 1024;
-__global__ void __launch_bounds__(WEQ_THREADS) k_weq(const Member* __restrict__ mem, int method) {
-    const Member& M = mem[blockIdx.x];
-    if (kview(M.ctl)->status != ST_RUN) return;
+//   2: corner BC (isos_utils.f90:104-118) of the viscous convolution.
+// The convolution leaves its result in the state buffer that the first attempt
+// will write, so every block reads the four corners there while all write weq
+// (one block per domain subtracting in place: 20.5 us at N = 256, now 4).
+__global__ void __launch_bounds__(PRE_THREADS) k_weq(const Member* __restrict__ mem, int method) {
+    const Member& M = mem[blockIdx.y];
+    const kptr<Ctl> ctl = kview(M.ctl);
+    if (ctl->status != ST_RUN) return;
     const int N = M.n;
     const size_t nn = (size_t)N * N;
     gmut<double> weq = gout<double>(M.weq);
-    if (method == 0) {
-        for (size_t c = threadIdx.x; c < nn; c += WEQ_THREADS) weq[c] = 0.0;
-        return;
+    gptr<double> cload = gin<double>(M.canom_load), raw = gin<double>(M.X[ctl->cur ^ 1]);
+    const double rho_um = kview(M.phys)->rho_uppermantle;
+    double cc = 0.0;
+    if (method == 2) cc = 0.25 * (raw[0] + raw[nn - 1] + raw[(size_t)(N - 1) * N] + raw[N - 1]);
+#pragma unroll
+    for (int it = 0; it < PRE_CELLS / PRE_THREADS; ++it) {
+        const size_t c = (size_t)blockIdx.x * PRE_CELLS + it * PRE_THREADS + threadIdx.x;
+        if (c >= nn) break;
+        weq[c] = method == 0 ? 0.0 : method == 1 ? -cload[c] / rho_um : raw[c] - cc;
     }
-    if (method == 1) {
-        const double rho_um = kview(M.phys)->rho_uppermantle;
-        gptr<double> cload = gin<double>(M.canom_load);
-        for (size_t c = threadIdx.x; c < nn; c += WEQ_THREADS) weq[c] = -cload[c] / rho_um;
-        return;
-    }
-    const double* raw = M.weq;
-    const double cc = 0.25 * (raw[0] + raw[nn - 1] + raw[(size_t)(N - 1) * N] + raw[N - 1]);
-    __syncthreads();
-    for (size_t c = threadIdx.x; c < nn; c += WEQ_THREADS) weq[c] = weq[c] - cc;
 }
 
 void launch_weq_input(const Member* d_mem, int nmem, int n, hipStream_t st) {
@@ -334,8 +332,9 @@ void launch_weq_input(const Member* d_mem, int nmem, int n, hipStream_t st) {
 }
 
 void launch_weq(const Member* d_mem, int nmem, int n, int method, hipStream_t st) {
-    (void)n;
-    hipLaunchKernelGGL(k_weq, dim3(nmem), dim3(WEQ_THREADS), 0, st, d_mem, method);
+    const size_t nn = (size_t)n * n;
+    hipLaunchKernelGGL(k_weq, dim3((unsigned)((nn + PRE_CELLS - 1) / PRE_CELLS), nmem), dim3(PRE_THREADS), 0, st,
+                       d_mem, method);
 }
 
 // The finalize kernels run once per update and domain, for domains that have
