@@ -174,16 +174,23 @@ void small_batch_shape(RhsShape& s, int nmem, bool tuned, const TunedShape& ts, 
                        const std::function<bool(int)>& inv_ok) {
     s.srow_rows = 0;
     s.threads_inv = 0;
-    // fewer blocks than CUs: fused blocks of 16 (or 4) rows, inverse blocks of threads_row
-    const bool few_rows = (long long)(s.n / 16) * nmem < 256, fewer_rows = (long long)(s.n / 4) * nmem < 256;
+    // blocks of `rows` rows too few for `want` of them (256: one per CU)
+    auto short_of = [&](int rows, int want) { return (long long)(s.n / rows) * nmem < want; };
     const bool few = (long long)(s.n / (2 * s.L)) * nmem < 256;
     if (s.fused && one_col_ok) {
         // (2-row blocks while 4-row ones would still leave CUs idle: one 256^2
         // domain's fused pass 6.25 us against 6.92; 16 rows in N threads where
         // the row blocks hold fewer threads than columns: one column per thread
         // keeps the march's window in registers)
+        // (8 rows while 16-row blocks would leave CUs idle, at 2^k while they
+        // would give each fewer than two: 4 of 512^2 24.6 us per attempt against
+        // 26.3 in 4-row blocks, 16 of 256^2 24.1 against 25.0 in 16-row ones; 12
+        // of 384^2 47.6 in 16-row blocks against 49.5)
         int r = tuned && ts.srow_rows ? ts.srow_rows
-                                      : (fewer_rows ? 2 : few_rows ? 4 : (s.threads_row < s.n ? 16 : 0));
+                : short_of(4, 256)    ? 2
+                : short_of(8, 256)    ? 4
+                : short_of(16, s.n == 384 ? 256 : 512) ? 8
+                                      : (s.threads_row < s.n ? 16 : 0);
         if (const char* e = std::getenv("FI_SROW_ROWS")) r = std::atoi(e);
         if (r == 2 || r == 4 || r == 8 || r == 16) s.srow_rows = r;
     }
@@ -228,9 +235,11 @@ int make_three_pass_shape(int n, int nmem, bool fp64, bool uniform, bool tuned, 
         };
         int best_c = 0;
         // the largest blocks that still give every CU one; no block below a
-        // wave when a wave-sized one exists (one 256^2 domain: 2 line pairs)
+        // wave when a wave-sized one exists (one 256^2 domain: 2 line pairs);
+        // FP64 at 4 line pairs, whose LDS lets four blocks share a CU (16 of
+        // 384^2: 75.3 us per attempt against 81.0 with 8)
         for (int C : {16, 8, 4, 2, 1}) {
-            if (!col_ok(C)) continue;
+            if (!col_ok(C) || (fp64 && C > 4)) continue;
             if (best_c && C * tpl < 64) break;
             best_c = C;
             if ((size_t)(n / (2 * C)) * nmem >= 256) break;
@@ -391,8 +400,9 @@ int make_three_pass_shape(int n, int nmem, bool fp64, bool uniform, bool tuned, 
 // 3 * 2^k) while launches and not bytes set the pace, measured per attempt
 // (two launches against three, mixed): one 64^2 domain 12.9 / 16.0 us, 256^2
 // 14.1 / 16.9, 512^2 17.9 / 19.8; 48 of 128^2 21.3 / 23.8, 12 of 256^2 23.0 /
-// 23.7 but 16 27.2 / 25.3; 6 of 384^2 31.1 / 35.5; 2 of 512^2 20.3 / 21.5 but 3
-// 29.8 / 26.8 and 2 in FP64 27.5 / 26.1.  A launch shape asked of the other
+// 23.7 but 16 27.2 / 25.0; 8 of 384^2 30.4 / 36.4 and 12 48.5 / 47.6 (FP64: 4 35.4 /
+// 38.8, 16 90.6 / 81.0); 2 of 512^2 20.3 / 21.5 but 3 29.8 / 26.8 and 2 in FP64
+// 27.5 / 26.1.  A launch shape asked of the other
 // kernels (environment, autotuner) keeps those; FI_TURN = 0 never, 2 wherever
 // the kernels exist (tests).
 //
@@ -400,7 +410,10 @@ int make_three_pass_shape(int n, int nmem, bool fp64, bool uniform, bool tuned, 
 // leaves CUs idle otherwise (one N = 320 domain 16.4 us against 17.8 with 8
 // per kt_col block), from 192 blocks on two and eight (2 of 512^2: 20.3 us
 // against 25.6; 8 of 320^2: 28.9 against 32.6).
-long long turn_cells(int n, bool fp64) { return n < 512 ? 12 << 16 : fp64 ? 1 << 18 : 1 << 19; }
+long long turn_cells(int n, bool fp64) {
+    if (n == 384 && !fp64) return 10 * 384 * 384;
+    return n < 512 ? 12 << 16 : fp64 ? 1 << 18 : 1 << 19;
+}
 
 void turn_shape(int n, int nmem, bool fp64, bool uniform, bool tuned, const TunedShape& ts, RhsShape& s) {
     s.turn = nullptr;
@@ -729,10 +742,15 @@ int ensure_sub(int k) {
     return 0;
 }
 
-// number of sub-batches for a batch of nmem domains (the autotuner's choice,
-// else 2 from 32 domains; FI_SUBBATCHES overrides)
-int sub_count(int n, bool fp64, int nmem) {
-    int k = nmem >= 32 ? 2 : 1;
+// number of sub-batches for a batch of nmem domains about to run `ahead`
+// attempts (the autotuner's choice, else 2 from 32 domains, and in FP64 off 2^k
+// from 1.5 million cells: 16 of 384^2 72.3 us per attempt against 81.0, 16 of 320^2
+// 69.5 against 78.7 -- while 8 of 512^2 lose, 56.7 against 50.6; FI_SUBBATCHES
+// overrides).  Splitting and joining the streams costs as much as a dozen
+// attempts gain.
+int sub_count(int n, bool fp64, int nmem, int ahead) {
+    const bool large = fp64 && (n & (n - 1)) != 0 && nmem >= 8 && (long long)n * n * nmem >= 3 << 19;
+    int k = nmem >= 32 || (large && ahead >= 16) ? 2 : 1;
     TunedShape ts;
     if (tuned_for(n, fp64, nmem, ts) && ts.K >= 1) k = ts.K;
     if (const char* e = std::getenv("FI_SUBBATCHES")) k = std::atoi(e);
@@ -967,7 +985,7 @@ int job_begin(UpdateJob& j) {
     if (again > need) need = again + 1.0;
     j.ahead = (int)std::min(256.0, std::max(1.0, need));
     // concurrent sub-batches only on the library stream (their streams are shared)
-    j.K = shape.method == 3 && j.st == g_stream && j.subbatch ? sub_count(n, h0.fp64, nmem) : 1;
+    j.K = shape.method == 3 && j.st == g_stream && j.subbatch ? sub_count(n, h0.fp64, nmem, j.ahead) : 1;
     if (j.K > 1) {
         int rc = ensure_sub(j.K);
         if (rc) return rc;
