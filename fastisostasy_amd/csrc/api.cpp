@@ -162,14 +162,12 @@ struct TunedShape {
 };
 
 // Rows per block of the fused stencil pass with one column per thread
-// (FI_SROW_ROWS = 4 | 8, or the tuned value; 0 keeps 2L rows): more,
+// (FI_SROW_ROWS = 2 | 4 | 8 | 16, or the tuned value; 0 keeps 2L rows): more,
 // shorter row blocks for small batches.  Block size of the inverse row pass
-// (FI_INV_THREADS, or the tuned value; 0 keeps threads_row).  Untuned, a
-// group whose 16-row fused blocks or default inverse blocks would not give
-// every CU one (256) takes 4-row (2-row) fused blocks and 64-thread inverse
-// blocks, the shapes the autotuner picks for a single 256^2 domain (0.95 ms
-// per 10-yr update against 1.16); larger groups whose row blocks hold fewer
-// threads than columns (FP64 at N = 512) take 16-row fused blocks of N threads.
+// (FI_INV_THREADS, or the tuned value; 0 keeps threads_row).  Untuned, the row
+// count follows from how many blocks there would be (below), and a group whose
+// default row blocks would not give every CU one (256) takes inverse blocks of
+// `def_inv` threads.
 void small_batch_shape(RhsShape& s, int nmem, bool tuned, const TunedShape& ts, bool one_col_ok, int def_inv,
                        const std::function<bool(int)>& inv_ok) {
     s.srow_rows = 0;
@@ -515,8 +513,9 @@ struct fi_isos {
     bool use_restart = false;    // a restart was read: the next init_state takes the restart branch
     double time_diag = 0, time_prog = 0;
     double last_t = 0, last_dt = 0;  // ode%t and ode%dt after the last update (host copy; 0 = unknown)
-    double last_span = 0;        // years and attempts of the last update (0: unknown)
-    long long last_attempts = 0, attempts_seen = 0;
+    struct Past { double span = 0; long long attempts = 0; };
+    Past past[4];                // years (0: unknown) and attempts of the last updates, newest first
+    long long attempts_seen = 0;
     int last_status = 0;         // status of the last update's instability and NaN checks
     char* arena = nullptr;
     size_t arena_bytes = 0;      // HBM footprint of the domain (one allocation)
@@ -971,18 +970,21 @@ int job_begin(UpdateJob& j) {
     // ended its previous update with, plus a margin for rejections; after each
     // readback job_more corrects the estimate.
     // A load that changes from one coupling step to the next cuts the step at
-    // the start of each update: then the last update of the same span is the
-    // better guess (N = 64 disc under varying ice: 6-7 attempts where the last dt
-    // promises one; a second round costs about 25 us, an unused attempt 4).
+    // the start of each update: then the most attempts among the last four
+    // updates of the same span are the better guess (N = 64 disc under varying
+    // ice: 6 to 9 attempts where the last dt promises one).  Four, because a
+    // second round costs about 25 us and an unused attempt 4: with the last
+    // update plus one instead, every other update took a second round.
     double need = 0.0, again = 0.0;
     for (int m = 0; m < nmem; ++m) {
         const fi_isos& h = *j.hs[m];
         const double span = j.t_of(m) - h.last_t;
         if (h.last_dt > 0.0) need = std::max(need, std::ceil(span / h.last_dt));
-        if (std::fabs(span - h.last_span) <= 1e-6 * span) again = std::max(again, (double)h.last_attempts);
+        for (const auto& p : h.past)
+            if (std::fabs(span - p.span) <= 1e-6 * span) again = std::max(again, (double)p.attempts);
     }
     if (need > 0.0) need += (double)first_round_margin();
-    if (again > need) need = again + 1.0;
+    need = std::max(need, again);
     j.ahead = (int)std::min(256.0, std::max(1.0, need));
     // concurrent sub-batches only on the library stream (their streams are shared)
     j.K = shape.method == 3 && j.st == g_stream && j.subbatch ? sub_count(n, h0.fp64, nmem, j.ahead) : 1;
@@ -1089,8 +1091,9 @@ int job_end(UpdateJob& j) {
         const CtlSummary& c = j.sb.h[m];
         fi_isos* h = j.hs[m];
         h->time_prog = j.t_of(m);
-        h->last_span = j.stepping && h->last_dt > 0.0 ? c.t - h->last_t : 0.0;
-        h->last_attempts = c.attempts - h->attempts_seen;
+        std::copy_backward(h->past, h->past + 3, h->past + 4);
+        h->past[0].span = j.stepping && h->last_dt > 0.0 ? c.t - h->last_t : 0.0;
+        h->past[0].attempts = c.attempts - h->attempts_seen;
         h->attempts_seen = c.attempts;
         h->last_t = c.t;
         h->last_dt = j.stepping ? c.dt : 0.0;
@@ -1729,7 +1732,7 @@ int fi_isos_init_state(fi_isos* h, const double* z_bed, const double* H_ice, dou
     // (the first update's launch estimate starts from dt_init)
     h->last_t = time;
     h->last_dt = h->par.dt_init;
-    h->last_span = 0.0;
+    for (auto& p : h->past) p = {};
     h->state_init = true;
     h->use_restart = false;
     return 0;
