@@ -61,6 +61,37 @@ template <typename T, int N, int LO> struct Turn {
     static_assert(THREADS <= 1024, "threads per block");
 };
 
+// The block's copy of the twiddle table, in 16-byte pieces: loaded early,
+// stored to LDS once the loads behind it have been issued.
+template <typename T, int N, int THREADS> struct TurnTw {
+    typedef T V __attribute__((ext_vector_type(16 / sizeof(T))));
+    static constexpr int U = 2 * N * (int)sizeof(T) / 16, Q = (U + THREADS - 1) / THREADS;
+    static_assert(2 * N * sizeof(T) % 16 == 0, "table of whole pieces");
+    V r[Q];
+    __device__ __forceinline__ TurnTw(const void* tw, int tid) {
+        gptr<V> g = gin<V>(tw);
+#pragma unroll
+        for (int k = 0; k < Q; ++k) r[k] = g[min(tid + THREADS * k, U - 1)];
+    }
+    __device__ __forceinline__ void store(cplx<T>* tw_l, int tid) const {
+#pragma unroll
+        for (int k = 0; k < Q; ++k)
+            if (tid + THREADS * k < U) ((V*)tw_l)[tid + THREADS * k] = r[k];
+    }
+};
+
+// Row spectrum between the two kernels (g2): column tiles of four (the last
+// one of two where 4 does not divide N), row pairs inside, the two rows of a
+// column side by side.  The column pass reads whole lines of its two columns'
+// tile -- in row-major order each of a wave's loads touched 32 cache lines --
+// and the row pass stores each row pair in one store.  Together with the
+// decision in a wave of its own: one 512^2 domain 18.9 -> 17.0 us per attempt,
+// 320^2 17.1 -> 16.5, 256^2 14.4 -> 13.8.
+template <int N> __device__ __forceinline__ int turn_at(int row, int c) {
+    const int w = N % 4 == 0 ? 4 : (c < N - 2 ? 4 : 2);
+    return (c & ~3) * N + (row >> 1) * (2 * w) + (c & 3) * 2 + (row & 1);
+}
+
 template <typename T, int N, int LO, bool UNI>
 __global__ void __launch_bounds__((Turn<T, N, LO>::THREADS)) kt_turn(const Member* __restrict__ mem,
                                                                    const void* __restrict__ twv, int first) {
@@ -101,13 +132,7 @@ __global__ void __launch_bounds__((Turn<T, N, LO>::THREADS)) kt_turn(const Membe
     auto crow = [](int r) { return r < 0 ? 0 : (r > N - 1 ? N - 1 : r); };
 
     // ---- loads that need no control block, in the order of use
-    constexpr int TWQ = (2 * N + THREADS - 1) / THREADS;
-    T twr[TWQ];
-    {
-        gptr<T> g = gin<T>(twv);
-#pragma unroll
-        for (int k = 0; k < TWQ; ++k) twr[k] = g[min(tid + THREADS * k, 2 * N - 1)];
-    }
+    TurnTw<T, N, THREADS> twr(twv, tid);
     cplx<T> v[PL::E];
     constexpr int NW = THREADS / 64, QPW = NW >= 4 ? 1 : (4 + NW - 1) / NW, CPL = (N + 63) / 64;
     double cq[QPW][CPL];
@@ -145,9 +170,7 @@ __global__ void __launch_bounds__((Turn<T, N, LO>::THREADS)) kt_turn(const Membe
     }
     __builtin_amdgcn_sched_barrier(0);
     const bool run = status == ST_RUN;
-#pragma unroll
-    for (int k = 0; k < TWQ; ++k)
-        if (tid + THREADS * k < 2 * N) ((T*)tw_l)[tid + THREADS * k] = twr[k];
+    twr.store(tw_l, tid);
     // kt_col left the decided control block in ctl_next; block 0 makes it
     // current (every block reads ctl_next) and marks this attempt's decision
     // as pending, after its last load
@@ -441,17 +464,17 @@ __global__ void __launch_bounds__((Turn<T, N, LO>::THREADS)) kt_turn(const Membe
         MixRow<T, N> xc((cplx<T>*)zreg, LINES, l);
         mix_fft<T, N>(v, t, on, tw_l, xc);
         if (!first) partials_store();
-        gmut<T> dst = gout<T>(M.g2);
+        using V2 = typename vec2<T>::type;
+        gmut<V2> dst = gout<V2>(M.g2);
         if (tid < N) {
 #pragma unroll
             for (int p = 0; p < LO; ++p) {
                 T ha, hb;
                 dht_pair(xc.at(p, tid), xc.at(p, tid ? N - tid : 0), ha, hb);
-                if (p >= own0) {
-                    const size_t at = (size_t)(row0 + 2 * p) * N + tid;
-                    dst[at] = ha;
-                    dst[at + N] = hb;
-                }
+                V2 o;
+                o.x = ha;
+                o.y = hb;
+                if (p >= own0) dst[turn_at<N>(row0 + 2 * p, tid) / 2] = o;
             }
         }
     }
@@ -461,7 +484,8 @@ __global__ void __launch_bounds__((Turn<T, N, LO>::THREADS)) kt_turn(const Membe
 // Column pass.  C complex lines (columns 2j, 2j+1) per block; the last block
 // of a domain transforms copies of its last line where C does not divide N/2.
 template <typename T, int N, int C> struct TurnCol {
-    static constexpr int THREADS = (C * MixPlan<N>::TPL + 63) / 64 * 64;
+    // waves of transforms, and one more that finds out whether they count
+    static constexpr int FFT = (C * MixPlan<N>::TPL + 63) / 64 * 64, THREADS = FFT + 64;
     static_assert(THREADS <= 1024, "threads per block");
     // column blocks of a domain, and one more block that only decides
     static constexpr int NB = (N / 2 + C - 1) / C;
@@ -504,68 +528,70 @@ __global__ void __launch_bounds__((TurnCol<T, N, C>::THREADS)) kt_col(const Memb
     const int status = c->status, pend = c->pending;
     const double c_dt = c->dt, c_t = c->t, c_tf = c->tf;
     extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ int go_s;
     cplx<T>* tw_l = (cplx<T>*)smem;
     const int tid = threadIdx.x, line = tid % C, t = tid / C;
-    const bool live = cblk * C + line < N / 2, on = t < PL::TPL;
+    const bool decider = __builtin_amdgcn_readfirstlane(tid) >= TurnCol<T, N, C>::FFT;
+    const bool live = cblk * C + line < N / 2, on = !decider && t < PL::TPL;
     const int ca = 2 * (live ? cblk * C + line : N / 2 - 1), tt = t < T0 ? t : 0;
-    // the previous attempt's partials first (the decision needs them), then
-    // twiddles, spectrum and kappa R; none of them depends on the control block
-    constexpr int NP = turn_reg8(N) ? N / 2 : N, PJ = (NP + 63) / 64;
-    typedef double d2v __attribute__((ext_vector_type(2)));
-    d2v pa[PJ];
-    {
+    // spectrum, twiddles, kappa R; none depends on the control block
+    using V2 = typename vec2<T>::type;
+    gptr<T> src = gin<T>(p_src);
+    gptr<V2> kR = gin<V2>(p_kr);
+    // (row, column pair) -> vector index of a row-major field
+    auto vec = [&](int row) { return ((unsigned)row * N + ca) / 2; };
+    V2 xk[R0];
+    cplx<T> v[PL::E];
+    double2 wa, wb;
+    // Run?  Yes for the first attempt of a round and after an accepted step
+    // that did not end the update; a rejected attempt keeps its right-hand
+    // side, which g1 holds.  The last wave finds out from the previous
+    // attempt's partials while the others transform (in line it was 1280 of
+    // 10800 cycles at N = 256).
+    if (decider) {
+        constexpr int NP = turn_reg8(N) ? N / 2 : N, PJ = (NP + 63) / 64;
+        typedef double d2v __attribute__((ext_vector_type(2)));
+        d2v pa[PJ];
         gptr<d2v> part = gin<d2v>(p_part);
         const int lane = tid & 63;
 #pragma unroll
         for (int j = 0; j < PJ; ++j) pa[j] = part[(size_t)min(lane + 64 * j, NP - 1) * 2];
-    }
-    constexpr int TWQ = (2 * N + THREADS - 1) / THREADS;
-    T twr[TWQ];
-    {
-        gptr<T> g = gin<T>(twv);
+        if (status != ST_RUN) return;
+        bool go = true;
+        if (pend) {
+            double amax = 0.0, s2 = 0.0;
 #pragma unroll
-        for (int k = 0; k < TWQ; ++k) twr[k] = g[min(tid + THREADS * k, 2 * N - 1)];
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    using V2 = typename vec2<T>::type;
-    gptr<V2> src = gin<V2>(p_src), kR = gin<V2>(p_kr);
-    // (row, column pair) -> vector index
-    auto vec = [&](int row) { return ((unsigned)row * N + ca) / 2; };
-    V2 xs[R0], xk[R0];
-#pragma unroll
-    for (int r = 0; r < R0; ++r) xs[r] = src[vec(tt + T0 * r)];
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int r = 0; r < R0; ++r) xk[r] = kR[vec(tt + T0 * r)];
-    const double2 wa = tw64[ca], wb = tw64[ca + 1];
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int k = 0; k < TWQ; ++k)
-        if (tid + THREADS * k < 2 * N) ((T*)tw_l)[tid + THREADS * k] = twr[k];
-    // Run?  Yes for the first attempt of a round and after an accepted step
-    // that did not end the update; a rejected attempt keeps its right-hand
-    // side, which g1 holds.
-    bool go = status == ST_RUN;
-    if (pend) {
-        const int lane = tid & 63;
-        double amax = 0.0, s2 = 0.0;
-#pragma unroll
-        for (int j = 0; j < PJ; ++j) {
-            const bool in = lane + 64 * j < NP;
-            amax = fmax(amax, in ? pa[j].x : 0.0);
-            s2 += in ? pa[j].y : 0.0;
+            for (int j = 0; j < PJ; ++j) {
+                const bool in = lane + 64 * j < NP;
+                amax = fmax(amax, in ? pa[j].x : 0.0);
+                s2 += in ? pa[j].y : 0.0;
+            }
+            amax = wave_max(amax);
+            s2 = wave_sum(s2);
+            go = step_goes_on(c_dt, c_t, c_tf, amax, s2, ph, N);
         }
-        amax = wave_max(amax);
-        s2 = wave_sum(s2);
-        go = __builtin_amdgcn_readfirstlane(step_goes_on(c_dt, c_t, c_tf, amax, s2, ph, N));
-    }
-    if (!go) return;
-    cplx<T> v[PL::E];
+        if (lane == 0) go_s = go;
+    } else {
+        TurnTw<T, N, TurnCol<T, N, C>::FFT> twr(twv, tid);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int r = 0; r < R0; ++r) v[r] = mk<T>(xs[r].x, xs[r].y);
+        for (int r = 0; r < R0; ++r) {
+            const int at = turn_at<N>(tt + T0 * r, ca);
+            v[r] = mk<T>(src[at], src[at + 2]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < R0; ++r) xk[r] = kR[vec(tt + T0 * r)];
+        wa = tw64[ca];
+        wb = tw64[ca + 1];
+        __builtin_amdgcn_sched_barrier(0);
+        if (status != ST_RUN) return;
+        twr.store(tw_l, tid);
+    }
     if constexpr (!PL::PLAIN0) __syncthreads();
     MixCol<T, N, C> xc((cplx<T>*)smem + N, line);
     mix_fft<T, N>(v, t, on, tw_l, xc);
+    if (!go_s) return;
     const bool has = on && t < T0;
     if (has) {
         // Hartley values and the spectral divide (lv_elva.f90:115)
@@ -636,7 +662,8 @@ template <typename T, int N>
 bool turn_n(const Member* d, int nmem, const RhsShape& s, hipStream_t st, int which) {
     const bool cols = which == 1 || which < 0, rows = which != 1;
     bool ok = true;
-    if (cols) ok = s.turn_C >= 8 ? turn_cols<T, N, 8>(d, nmem, s, st, which) : turn_cols<T, N, 2>(d, nmem, s, st, which);
+    constexpr int CW = MixPlan<N>::TPL <= 120 ? 8 : 4;   // (with the deciding wave, at most 1024 threads)
+    if (cols) ok = s.turn_C >= 8 ? turn_cols<T, N, CW>(d, nmem, s, st, which) : turn_cols<T, N, 2>(d, nmem, s, st, which);
     if (rows && ok)
         ok = s.uniform ? (s.turn_LO == 1 ? turn_rows<T, N, 1, true>(d, nmem, s, st, which)
                                          : turn_rows<T, N, 2, true>(d, nmem, s, st, which))
