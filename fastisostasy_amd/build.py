@@ -18,6 +18,9 @@ FLAGS = [
     # packed FP32 instructions are disabled on purpose: some of their forms
     # have returned wrong results on this hardware without raising an error
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # kernel arguments preloaded into scalar registers: the first loads of a
+    # kernel need not wait for its argument segment
+    "-mllvm", "-amdgpu-kernarg-preload-count=14",
     "-Wall", "-Wno-unused-function", "-Wno-unused-variable",
 ]
 

@@ -483,7 +483,6 @@ int make_conv_shape(int n, bool fp64, ConvShape& s) {
     return 0;
 }
 
-size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 }  // namespace
 
@@ -819,7 +818,7 @@ bool same_shape(const RhsShape& a, const RhsShape& b) {
            a.fused == b.fused && a.row_tiles == b.row_tiles && a.srow_rows == b.srow_rows &&
            a.threads_inv == b.threads_inv && a.tw == b.tw && a.tw64 == b.tw64 &&
            a.plan.n == b.plan.n && a.plan.nf == b.plan.nf && a.method == b.method && a.dt_method == b.dt_method && a.turn == b.turn &&
-           a.turn_C == b.turn_C && a.turn_LO == b.turn_LO;
+           a.turn_C == b.turn_C && a.turn_LO == b.turn_LO && a.solo == b.solo;
 }
 
 int attempt_graph(const Member* d, int nmem, const RhsShape& s, hipStream_t st, hipGraphExec_t* out) {
@@ -1428,13 +1427,14 @@ static int create_impl(const fi_params* p, int nx_ice, int ny_ice, double dx, do
         if (rc) { delete h; return rc; }
     }
     const size_t rp = h->fp64 ? 8 : 4;
-    h->part_blocks = (int)std::max<size_t>((nn + 1023) / 1024, (size_t)n);
+    h->part_blocks = (int)partial_blocks(n);
+    h->shape.solo = true;
 
-    // ---- arena layout
-    size_t off = 0;
+    // ---- arena layout: the Member and what the attempts touch, then the rest
+    const HotLayout hot = hot_layout(n, rp);
+    size_t off = hot.end;
     auto take = [&](size_t bytes) { size_t o = off; off += align256(bytes); return o; };
     const size_t f64 = nn * 8;
-    size_t oX0 = take(f64), oX1 = take(f64), oW = take(f64), odw = take(f64);
     size_t oz = take(f64), ozss = take(f64), odz = take(f64), owe = take(f64), oH = take(f64), oHaf = take(f64);
     size_t ocm = take(f64), ocf = take(f64), ocl = take(f64), oci = take(f64);
     size_t ozr = take(f64), ozssr = take(f64), ohafr = take(f64), ohr = take(f64), owr = take(f64), ower = take(f64),
@@ -1443,10 +1443,6 @@ static int create_impl(const fi_params* p, int nx_ice, int ny_ice, double dx, do
     if (!h->uniform) { oA = take(f64); odxm = take(f64); oK2 = take(f64); }
     size_t omask = take(nn), omaskr = take(nn);
     size_t oHin = take((size_t)nx_ice * ny_ice * 8);
-    size_t oD = take(nn * rp), oeta = take(nn * rp), okR = take(nn * rp), ocfr = take(nn * rp), og1 = take(nn * rp),
-           og2 = take(nn * rp);
-    // partials: 4 values per block for the attempt kernels, 5 for the finalize reduction
-    size_t ocor = take((size_t)n * 4 * 8), opart = take((size_t)h->part_blocks * 5 * 8);
     size_t oee = take(f64), okap = take(f64), oR = take(f64), oHe = take(f64), oDd = take(f64);
     size_t oscr = take(f64 + 64);
     size_t oweq = (p->method != 3) ? take(f64) : 0;
@@ -1454,8 +1450,6 @@ static int create_impl(const fi_params* p, int nx_ice, int ny_ice, double dx, do
     size_t ocw = 0, oFGE = 0, oFGN = 0, oFGV = 0;
     if (h->has_conv) { ocw = take(2 * (size_t)n * hc); oFGE = take(2 * (size_t)n * hc); oFGN = take(2 * (size_t)n * hc); }
     if (p->method == 2) oFGV = take(2 * (size_t)n * hc);
-    size_t octl = take(sizeof(Ctl)), octl2 = take(sizeof(Ctl)), ophys = take(sizeof(PhysDev)),
-           omem = take(sizeof(Member));
     if (hipMalloc(&h->arena, off) != hipSuccess) { delete h; return fail(FI_E_HIP, "hipMalloc arena (%zu bytes)", off); }
     h->arena_bytes = off;
     HIPCHK(hipMemsetAsync(h->arena, 0, off, g_stream));
@@ -1464,7 +1458,8 @@ static int create_impl(const fi_params* p, int nx_ice, int ny_ice, double dx, do
     char* a = h->arena;
     Member& M = h->hm;
     M.n = n; M.icrop1 = h->icrop1; M.jcrop1 = h->jcrop1; M.nx_ice = nx_ice; M.ny_ice = ny_ice;
-    M.X[0] = (double*)(a + oX0); M.X[1] = (double*)(a + oX1); M.W = (double*)(a + oW); M.dwdt = (double*)(a + odw);
+    M.X[0] = (double*)(a + hot.X0); M.X[1] = (double*)(a + hot.X1);
+    M.W = (double*)(a + hot.W); M.dwdt = (double*)(a + hot.dwdt);
     M.z_bed = (double*)(a + oz); M.z_ss = (double*)(a + ozss); M.dz_ss = (double*)(a + odz); M.we = (double*)(a + owe);
     M.Hice = (double*)(a + oH); M.Haf = (double*)(a + oHaf); M.canom_mantle = (double*)(a + ocm);
     M.canom_full = (double*)(a + ocf); M.canom_load = (double*)(a + ocl); M.conv_in = (double*)(a + oci);
@@ -1474,12 +1469,12 @@ static int create_impl(const fi_params* p, int nx_ice, int ny_ice, double dx, do
     if (!h->uniform) { M.A = (double*)(a + oA); M.dxm = (double*)(a + odxm); M.K2 = (double*)(a + oK2); }
     M.mask = (uint8_t*)(a + omask); M.mask_ref = (uint8_t*)(a + omaskr);
     M.H_in = (double*)(a + oHin);
-    M.D = a + oD; M.eta = a + oeta; M.kR = a + okR; M.cfull = a + ocfr; M.g1 = a + og1; M.g2 = a + og2;
-    M.corners = (double*)(a + ocor); M.partials = (double*)(a + opart);
-    M.ctl = (Ctl*)(a + octl); M.ctl_next = (Ctl*)(a + octl2); M.phys = (PhysDev*)(a + ophys);
+    M.D = a + hot.D; M.eta = a + hot.eta; M.kR = a + hot.kR; M.cfull = a + hot.cfull; M.g1 = a + hot.g1; M.g2 = a + hot.g2;
+    M.corners = (double*)(a + hot.corners); M.partials = (double*)(a + hot.partials);
+    M.ctl = (Ctl*)(a + hot.ctl); M.ctl_next = (Ctl*)(a + hot.ctl_next); M.phys = (PhysDev*)(a + hot.phys);
     M.bsl_lead = 1;
     M.bsl_next = -1;
-    h->d_mem = (Member*)(a + omem);
+    h->d_mem = (Member*)a;
     h->eta_eff = (double*)(a + oee); h->kappa = (double*)(a + okap); h->R = (double*)(a + oR);
     h->He = (double*)(a + oHe); h->Dd = (double*)(a + oDd);
     double* scratch = (double*)(a + oscr);
@@ -1802,8 +1797,10 @@ int fi_isos_update_noalloc(fi_isos* h, const double* H_ice, double time, fi_bsl*
     HIPCHK(hipMemcpyAsync(d_mem, &M, sizeof(Member), hipMemcpyHostToDevice, g_stream));
     HIPCHK(hipMemcpyAsync(h->hm.H_in, H_ice, sizeof(double) * h->nx_ice * h->ny_ice, hipMemcpyHostToDevice, g_stream));
     std::vector<fi_isos*> hs{h};
+    RhsShape shape = h->shape;
+    shape.solo = false;   // (the Member's copy in the scratch names other work arrays)
     // plain launches: capturing an attempt graph would allocate
-    return run_update(hs, d_mem, h->shape, h->sb, time, true, nullptr, false);
+    return run_update(hs, d_mem, shape, h->sb, time, true, nullptr, false);
 }
 
 static const double* field_ptr(fi_isos* h, int f, bool& is_mask, int& bit) {

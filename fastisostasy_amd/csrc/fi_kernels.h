@@ -39,6 +39,7 @@ struct RhsShape {
     TurnFn turn;      // not null: attempts run as kt_col, kt_turn (rhs_turn.hpp)
     int turn_C;       // line pairs per kt_col block (2 or 8)
     int turn_LO;      // line pairs per kt_turn block (1 or 2)
+    bool solo;        // one domain, launched through the Member in its own arena (HotLayout)
 };
 
 // The three passes of a convolution of one length and precision (conv_mix.hpp):

@@ -1,5 +1,6 @@
 // fi_types.h -- plain structs shared by host and device code of the HIP library.
 #pragma once
+#include <stddef.h>
 #include <stdint.h>
 
 namespace fi {
@@ -121,5 +122,40 @@ struct Member {
     int bsl_lead, bsl_next;
     double tf_req;               // per-domain target time of a serving round
 };
+
+// Where a domain's arena keeps what the attempt kernels touch, as offsets from
+// its Member (the arena's first bytes): a launch for one domain finds its
+// arrays from the Member's address alone, with no descriptor to load first.
+constexpr size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
+constexpr size_t partial_blocks(int n) {
+    const size_t nb = ((size_t)n * n + 1023) / 1024;
+    return nb > (size_t)n ? nb : (size_t)n;
+}
+struct HotLayout { size_t ctl, ctl_next, phys, X0, X1, W, dwdt, D, eta, kR, cfull, g1, g2, corners, partials, end; };
+// rp: bytes of the RHS precision
+constexpr HotLayout hot_layout(int n, size_t rp) {
+    HotLayout l{};
+    size_t o = align256(sizeof(Member));
+    const size_t f = align256((size_t)n * n * 8), r = align256((size_t)n * n * rp);
+    l.ctl = o; o += align256(sizeof(Ctl));
+    l.ctl_next = o; o += align256(sizeof(Ctl));
+    l.phys = o; o += align256(sizeof(PhysDev));
+    l.X0 = o; o += f;
+    l.X1 = o; o += f;
+    l.W = o; o += f;
+    l.dwdt = o; o += f;
+    l.D = o; o += r;
+    l.eta = o; o += r;
+    l.kR = o; o += r;
+    l.cfull = o; o += r;
+    l.g1 = o; o += r;
+    l.g2 = o; o += r;
+    // per-column corner terms; partials: 4 values per block for the attempt
+    // kernels, 5 for the finalize reduction
+    l.corners = o; o += align256((size_t)n * 4 * 8);
+    l.partials = o; o += align256(partial_blocks(n) * 5 * 8);
+    l.end = o;
+    return l;
+}
 
 }  // namespace fi

@@ -221,13 +221,14 @@ template <> struct vec2<float> { typedef float type __attribute__((ext_vector_ty
 template <> struct vec2<double> { typedef double type __attribute__((ext_vector_type(2))); };
 
 // (member, block-within-member) for a grid (blocks per member, members)
-__device__ __forceinline__ void xcd_order(int& member, int& blk) {
-    const int per = gridDim.x, total = gridDim.x * gridDim.y;
+__device__ __forceinline__ void xcd_order(int per, int nmem, int& member, int& blk) {
+    const int total = per * nmem;
     int b = blockIdx.x + per * blockIdx.y;
     if ((total & 7) == 0) b = (b & 7) * (total >> 3) + (b >> 3);
     member = b / per;
     blk = b % per;
 }
+__device__ __forceinline__ void xcd_order(int& member, int& blk) { xcd_order(gridDim.x, gridDim.y, member, blk); }
 
 // Reduce the per-thread row statistics of two rows over the TPL threads of a
 // line with a fixed butterfly (lines wider than a wave combine their wave

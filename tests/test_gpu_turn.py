@@ -71,3 +71,22 @@ def test_turn_bitwise(n, prec, distorted, members, monkeypatch):
         for f in ("w", "dwdt", "z_bed"):
             assert np.array_equal(r[f], g[f]), (f, np.abs(r[f] - g[f]).max())
     assert np.abs(got[0]["w"]).max() > 0 and got[0]["attempts"] > got[0]["accepts"] > 4
+
+
+@pytest.mark.parametrize("n,prec,distorted", [(50, "mixed", False), (96, "fp64", True), (250, "mixed", True),
+                                              (256, "fp64", False), (384, "mixed", False)])
+def test_arena_and_descriptor_addresses(n, prec, distorted, monkeypatch):
+    """A single domain's launches find its arrays by their offsets from its
+    Member; a group's (here of one) by the descriptor's pointers."""
+    print(f"case: addresses N={n} {prec} distorted={distorted}", flush=True)
+    for k in SHAPE_ENV:
+        monkeypatch.delenv(k, raising=False)
+    ref = _run(n, prec, distorted, 1)[0]
+    h, b, H = _make(n, prec, distorted, 0)
+    bat = G.Batch([h])
+    for t in (2.0, 4.5):
+        bat.update(t, [b], [H])
+    bat.close()
+    assert h.scalar("t") == ref["t"] and h.scalar("attempts") == ref["attempts"] > 4
+    for f in ("w", "dwdt", "z_bed"):
+        assert np.array_equal(h.full(f), ref[f]), f
