@@ -23,6 +23,15 @@ __device__ __forceinline__ double attempt_dt(const Ctl& c, const PhysDev& ph) {
 __device__ __forceinline__ double kdiv(double h, double kr) { return h / kr; }
 __device__ __forceinline__ float kdiv(float h, float rkr) { return h * rkr; }
 
+// a / b for a divisor whose correctly rounded reciprocal y is at hand: the
+// quotient a y corrected once by its exact remainder, which rounds correctly
+// (P. Markstein, IBM J. Res. Dev. 34, 1990); the fix-up gives infinities, NaN
+// and zeros the division's results.  Four instructions against about a dozen.
+__device__ __forceinline__ double over_known(double a, double b, double y) {
+    const double q = a * y, r = __builtin_fma(-q, b, a);
+    return __builtin_amdgcn_div_fixup(__builtin_fma(r, y, q), b, a);
+}
+
 // Scalar-cache views of the control block and the physics scalars.  Both are
 // read-only while an attempt pass runs (k_decide, a separate launch, writes
 // Ctl), so their fields load with SMEM into SGPRs rather than with one vector

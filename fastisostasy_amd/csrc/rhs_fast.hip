@@ -734,7 +734,7 @@ __global__ void __launch_bounds__(THREADS) kf_row_inv(const Member* __restrict__
         const double S = (double)(float)((double)N * (double)N), rS = 1.0 / S;
         auto scl = [&](double x) {
             if constexpr (IsPow2<N>::value) return x * rS;
-            else return x / S;
+            else return over_known(x, S, rS);
         };
         cplx<T> m[E];
 #pragma unroll

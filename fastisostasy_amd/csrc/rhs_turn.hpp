@@ -320,7 +320,7 @@ __global__ void __launch_bounds__((Turn<T, N, LO>::THREADS)) kt_turn(const Membe
         const double S = (double)(float)((double)N * (double)N), rS = 1.0 / S;
         auto scl = [&](double x) {
             if constexpr ((N & (N - 1)) == 0) return x * rS;
-            else return x / S;
+            else return over_known(x, S, rS);
         };
         // x(1,1) + x(nx,ny) + x(1,ny) + x(nx,1)  (isos_utils.f90:116)
         const double cc = 0.25 * (scl(qs[0]) + scl(qs[3]) + scl(qs[2]) + scl(qs[1]));
