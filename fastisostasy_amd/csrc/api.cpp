@@ -393,24 +393,30 @@ int make_three_pass_shape(int n, int nmem, bool fp64, bool uniform, bool tuned, 
 
 // Two-launch attempts (rhs_turn.hpp) for this group?  At the general lengths
 // always: they replace five launches of the mixed-radix LDS kernels (one
-// N = 320 domain, mixed: 16.4 us per attempt against 59.5; 64 of 200^2: 60.5
+// N = 320 domain, mixed: 15.6 us per attempt against 59.5; 64 of 200^2: 51.6
 // against 155).  At the lengths of the three-launch register kernels (2^k,
 // 3 * 2^k) while launches and not bytes set the pace, measured per attempt
-// (two launches against three, mixed): one 64^2 domain 12.9 / 16.0 us, 256^2
-// 14.1 / 16.9, 512^2 17.9 / 19.8; 48 of 128^2 21.3 / 23.8, 12 of 256^2 23.0 /
-// 23.7 but 16 27.2 / 25.0; 8 of 384^2 30.4 / 36.4 and 12 48.5 / 47.6 (FP64: 4 35.4 /
-// 38.8, 16 90.6 / 81.0); 2 of 512^2 20.3 / 21.5 but 3 29.8 / 26.8 and 2 in FP64
-// 27.5 / 26.1.  A launch shape asked of the other
-// kernels (environment, autotuner) keeps those; FI_TURN = 0 never, 2 wherever
-// the kernels exist (tests).
+// (two launches against three, mixed): one 256^2 domain 13.3 / 16.9 us, 512^2
+// 16.5 / 19.8; 48 of 128^2 21.9 / 21.9, 12 of 256^2 23.6 / 23.5, 13 27.4 / 24.6
+// (FP64: 8 20.8 / 22.5, 10 31.3 / 29.9); 28 of 192^2 31.2 / 41.8 and 32 46.3 /
+// 45.7 (FP64: 28 40.1 / 52.3); 13 of 384^2 47.2 / 50.3 and 14 51.3 / 51.0
+// (FP64: 8 48.8 / 50.3, 16 90.6 / 81.0); 2 of 512^2 20.1 / 21.4 but 3 30.7 /
+// 27.6 and 2 in FP64 27.7 / 26.5.  A launch shape asked of the other kernels
+// (environment, autotuner) keeps those; FI_TURN = 0 never, 2 wherever the
+// kernels exist (tests).
 //
-// Blocks: one line pair per kt_turn block and two per kt_col block while that
-// leaves CUs idle otherwise (one N = 320 domain 16.4 us against 17.8 with 8
-// per kt_col block), from 192 blocks on two and eight (2 of 512^2: 20.3 us
-// against 25.6; 8 of 320^2: 28.9 against 32.6).
+// Blocks: one line pair per kt_turn block while that leaves CUs idle otherwise
+// (two from 192 half-pairs of lines on, 160 in FP64: 2 of 512^2 20.1 us
+// against 21.4, 2 of 320^2 in FP64 19.6 against 20.6, but one 512^2 domain 16.9
+// against 18.1), two line pairs per kt_col block up to 512 of them (8 of 256^2
+// 16.6 us against 18.5 with eight), eight beyond (12 of 256^2 23.5 against
+// 25.8) and, up to N = 128, where two line pairs fill half a wave, from 192 on
+// (16 of 128^2 beside other groups: 1.4% of a serving mix of 40 domains).
 long long turn_cells(int n, bool fp64) {
-    if (n == 384 && !fp64) return 10 * 384 * 384;
-    return n < 512 ? 12 << 16 : fp64 ? 1 << 18 : 1 << 19;
+    if (n == 192) return 28 * 192 * 192;
+    if (n == 384) return (fp64 ? 8 : 13) * 384 * 384;
+    if (n == 512) return fp64 ? 1 << 18 : 1 << 19;
+    return fp64 ? 8 << 16 : 12 << 16;
 }
 
 void turn_shape(int n, int nmem, bool fp64, bool uniform, bool tuned, const TunedShape& ts, RhsShape& s) {
@@ -425,8 +431,8 @@ void turn_shape(int n, int nmem, bool fp64, bool uniform, bool tuned, const Tune
     if (tuned && (ts.threads_row || ts.C || ts.row_tiles || ts.gL || ts.gC || ts.srow_rows || ts.threads_inv)) return;
     const long long blocks = (long long)(n / 4) * nmem;
     if (s.fast && want != 2 && (long long)n * n * nmem > turn_cells(n, fp64)) return;
-    s.turn_C = blocks >= 192 ? 8 : 2;
-    s.turn_LO = blocks >= 192 ? 2 : 1;
+    s.turn_C = blocks > (n <= 128 ? 191 : 512) ? 8 : 2;
+    s.turn_LO = blocks >= (fp64 ? 160 : 192) ? 2 : 1;
     // FI_TURN_LO = 1 | 2, FI_TURN_C = 2 | 8 override the blocks (tuning)
     if (const char* e = std::getenv("FI_TURN_LO")) s.turn_LO = std::atoi(e) == 1 ? 1 : 2;
     if (const char* e = std::getenv("FI_TURN_C")) s.turn_C = std::atoi(e) == 8 ? 8 : 2;
