@@ -233,7 +233,10 @@ template <> struct vec2<double> { typedef double type __attribute__((ext_vector_
 __device__ __forceinline__ void xcd_order(int per, int nmem, int& member, int& blk) {
     const int total = per * nmem;
     int b = blockIdx.x + per * blockIdx.y;
-    if ((total & 7) == 0) b = (b & 7) * (total >> 3) + (b >> 3);
+    // block b runs on XCD b % 8: XCD x takes the x-th of eight consecutive runs
+    // of total / 8 blocks, the first total % 8 of them one longer
+    const int x = b & 7, rest = total & 7;
+    b = x * (total >> 3) + (x < rest ? x : rest) + (b >> 3);
     member = b / per;
     blk = b % per;
 }

@@ -535,7 +535,13 @@ __global__ void __launch_bounds__((TurnCol<T, N, C>::THREADS)) kt_col(const Memb
     constexpr int THREADS = TurnCol<T, N, C>::THREADS, R0 = PL::R0, T0 = PL::T0;
     // a domain's column blocks on one XCD: neighbours share 128-byte lines
     int mi, cblk;
-    xcd_order(TurnCol<T, N, C>::NB + 1, nmem, mi, cblk);
+    // -- but spread over all of them while there are fewer than nine blocks for
+    // each: the few lines then come through eight L2 caches at once (one 512^2
+    // domain 16.5 -> 16.3 us per attempt in order, 6 of 300^2 30.7 -> 28.8, 2 of
+    // 512^2 23.1 -> 21.4; one 256^2 13.2 -> 13.3, N = 64 coupling step 104 -> 106)
+    mi = blockIdx.y;
+    cblk = blockIdx.x;
+    if ((TurnCol<T, N, C>::NB + 1) * nmem >= 72) xcd_order(TurnCol<T, N, C>::NB + 1, nmem, mi, cblk);
     const TurnPtrs P = turn_ptrs<T, N>(mem, mi, solo);
     const void *p_src = P.g2, *p_kr = P.kR;
     const double* const p_part = P.partials;
