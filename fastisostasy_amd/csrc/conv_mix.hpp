@@ -46,14 +46,7 @@ __device__ __forceinline__ void conv_rows(int j, int pair, int& ra, int& rb) {
 }
 
 template <typename T, int THREADS, int M> __device__ __forceinline__ void conv_twiddles(cplx<T>* tw_l, const void* twv) {
-    constexpr int Q = (2 * M + THREADS - 1) / THREADS;
-    gptr<T> g = gin<T>(twv);
-    T r[Q];
-#pragma unroll
-    for (int k = 0; k < Q; ++k) r[k] = g[min((int)threadIdx.x + THREADS * k, 2 * M - 1)];
-#pragma unroll
-    for (int k = 0; k < Q; ++k)
-        if ((int)threadIdx.x + THREADS * k < 2 * M) ((T*)tw_l)[threadIdx.x + THREADS * k] = r[k];
+    MixTable<T, M, THREADS>(twv, threadIdx.x).store(tw_l, threadIdx.x);
 }
 
 template <typename T, int M>
@@ -107,10 +100,15 @@ __global__ void __launch_bounds__((ConvMix<T, M>::TC)) cm_cols(const Member* __r
     using CM = ConvMix<T, M>;
     using PL = MixPlan<M>;
     constexpr int N = CM::N, H = CM::H, R0 = PL::R0, T0 = PL::T0, C = CM::CB;
-    const Member& Mb = mem[blockIdx.y];
+    // neighbouring columns share 128-byte lines: one XCD's blocks take a run of
+    // them (FP64, 16 of 384^2: 1594 -> 1566 us per coupling step; one N = 512 355 ->
+    // 342), but blocks fewer than nine per XCD spread over all
+    int mi = blockIdx.y, cblk = blockIdx.x;
+    if (gridDim.x * gridDim.y >= 72) xcd_order(mi, cblk);
+    const Member& Mb = mem[mi];
     extern __shared__ __align__(16) unsigned char smem[];
     cplx<T>* tw_l = (cplx<T>*)smem;
-    const int tid = threadIdx.x, line = tid % C, t = tid / C, kx = blockIdx.x * C + line;
+    const int tid = threadIdx.x, line = tid % C, t = tid / C, kx = cblk * C + line;
     const bool on = t < PL::TPL, has = t < T0 && kx < H;
     const int kc = kx < H ? kx : H - 1, tt = t < T0 ? t : 0;
     using V2 = typename vec2<T>::type;
@@ -198,7 +196,11 @@ __global__ void __launch_bounds__((ConvMix<T, M>::TR)) cm_rows_c2r(const Member*
     if constexpr (!PL::PLAIN0) __syncthreads();
     MixRow<T, M> xc(tw_l + M, LB, line < LB ? line : 0);
     mix_fft<T, M>(v, t, on, tw_l, xc);
-    const double scale = (double)M * (double)M;
+    const double scale = (double)M * (double)M, rscale = 1.0 / scale;
+    auto scl = [&](double x) {
+        if constexpr ((M & (M - 1)) == 0) return x * rscale;
+        else return over_known(x, scale, rscale);
+    };
     // (the viscous convolution goes to the state buffer that is free until the first attempt, k_weq)
     gmut<double> out = gout<double>((which == 0) ? Mb.we : (which == 1) ? Mb.dz_ss : Mb.X[Mb.ctl->cur ^ 1]);
     for (int q = tid; q < LB * N; q += CM::TR) {
@@ -208,8 +210,8 @@ __global__ void __launch_bounds__((ConvMix<T, M>::TR)) cm_rows_c2r(const Member*
         conv_rows(j0 + l, pair, a, b);
         // conj of the FFT: real part = row a, -(imag) = row b
         const cplx<T> z = xc.at(l, i + CM::C0);
-        out[(size_t)a * N + i] = (double)z.x / scale - cc;
-        out[(size_t)b * N + i] = -(double)z.y / scale - cc;
+        out[(size_t)a * N + i] = scl((double)z.x) - cc;
+        out[(size_t)b * N + i] = -scl((double)z.y) - cc;
     }
 }
 

@@ -17,6 +17,7 @@
 #include <type_traits>
 
 #include "fft_reg.hpp"
+#include "rhs_common.hpp"
 
 namespace fi {
 
@@ -81,6 +82,25 @@ template <int N> struct MixPlan {
     // be published before the first exchange's barrier does so
     static constexpr bool PLAIN0 = S.first[1] - S.first[0] == 1 && S.ng > 1;
     static constexpr int product(int a, int b) { return a >= b ? 1 : S.rad[a] * product(a + 1, b); }
+};
+
+// The block's copy of the twiddle table, in 16-byte pieces: loaded early,
+// stored to LDS once the loads behind it have been issued.
+template <typename T, int N, int THREADS> struct MixTable {
+    typedef T V __attribute__((ext_vector_type(16 / sizeof(T))));
+    static constexpr int U = 2 * N * (int)sizeof(T) / 16, Q = (U + THREADS - 1) / THREADS;
+    static_assert(2 * N * sizeof(T) % 16 == 0, "table of whole pieces");
+    V r[Q];
+    __device__ __forceinline__ MixTable(const void* tw, int tid) {
+        gptr<V> g = gin<V>(tw);
+#pragma unroll
+        for (int k = 0; k < Q; ++k) r[k] = g[min(tid + THREADS * k, U - 1)];
+    }
+    __device__ __forceinline__ void store(cplx<T>* tw_l, int tid) const {
+#pragma unroll
+        for (int k = 0; k < Q; ++k)
+            if (tid + THREADS * k < U) ((V*)tw_l)[tid + THREADS * k] = r[k];
+    }
 };
 
 // Radix-3 butterfly of the N = 3 * 2^k register engine (fft_reg.hpp): the same

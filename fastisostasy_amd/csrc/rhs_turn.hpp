@@ -61,25 +61,6 @@ template <typename T, int N, int LO> struct Turn {
     static_assert(THREADS <= 1024, "threads per block");
 };
 
-// The block's copy of the twiddle table, in 16-byte pieces: loaded early,
-// stored to LDS once the loads behind it have been issued.
-template <typename T, int N, int THREADS> struct TurnTw {
-    typedef T V __attribute__((ext_vector_type(16 / sizeof(T))));
-    static constexpr int U = 2 * N * (int)sizeof(T) / 16, Q = (U + THREADS - 1) / THREADS;
-    static_assert(2 * N * sizeof(T) % 16 == 0, "table of whole pieces");
-    V r[Q];
-    __device__ __forceinline__ TurnTw(const void* tw, int tid) {
-        gptr<V> g = gin<V>(tw);
-#pragma unroll
-        for (int k = 0; k < Q; ++k) r[k] = g[min(tid + THREADS * k, U - 1)];
-    }
-    __device__ __forceinline__ void store(cplx<T>* tw_l, int tid) const {
-#pragma unroll
-        for (int k = 0; k < Q; ++k)
-            if (tid + THREADS * k < U) ((V*)tw_l)[tid + THREADS * k] = r[k];
-    }
-};
-
 // Row spectrum between the two kernels (g2): column tiles of four (the last
 // one of two where 4 does not divide N), row pairs inside, the two rows of a
 // column side by side.  The column pass reads whole lines of its two columns'
@@ -166,7 +147,7 @@ __global__ void __launch_bounds__((Turn<T, N, LO>::THREADS)) kt_turn(const Membe
     auto crow = [](int r) { return r < 0 ? 0 : (r > N - 1 ? N - 1 : r); };
 
     // ---- loads that need no control block, in the order of use
-    TurnTw<T, N, THREADS> twr(twv, tid);
+    MixTable<T, N, THREADS> twr(twv, tid);
     cplx<T> v[PL::E];
     constexpr int NW = THREADS / 64, QPW = NW >= 4 ? 1 : (4 + NW - 1) / NW, CPL = (N + 63) / 64;
     double cq[QPW][CPL];
@@ -612,7 +593,7 @@ __global__ void __launch_bounds__((TurnCol<T, N, C>::THREADS)) kt_col(const Memb
         }
         if (lane == 0) go_s = go;
     } else {
-        TurnTw<T, N, TurnCol<T, N, C>::FFT> twr(twv, tid);
+        MixTable<T, N, TurnCol<T, N, C>::FFT> twr(twv, tid);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int r = 0; r < R0; ++r) {
