@@ -24,12 +24,14 @@ template <typename T, int M> struct ConvMix {
     static constexpr int N = M / 2, H = N + 1, C0 = N / 2 - 1;   // crop start (convolutions.f90:34-39), N even
     // rows: lines per block for about 256 threads;  columns: measured (us, one
     // domain / 16): FP64 M = 1024 with 4 columns and one exchange buffer 13.1 /
-    // 140 (two columns and two buffers: 21.9 / 216, one block per CU), M = 768 9.5
-    // / 71 (9.6 / 89); FP32 M = 1024 with 8 columns and one buffer 9.3 / 74 (4 and
-    // two 9.6 / 110); short FP32 lines with 4 and two buffers 6.2 / 19.3
+    // 140 (two columns and two buffers: 21.9 / 216, one block per CU); a coupling
+    // step with two columns and one buffer: FP64 N = 153 192 us against 197, 240
+    // 194.5 / 196.5, 16 of 384^2 1440 / 1465, but N = 512 347 / 342; FP32 M = 1024
+    // with 8 columns and one buffer 9.3 / 74 (4 and two 9.6 / 110); short FP32
+    // lines with 4 and two buffers 6.2 / 19.3
     static constexpr int LB = PL::TPL >= 128 ? 2 : 256 / PL::TPL > 8 ? 8 : 256 / PL::TPL;
     // (M = 1000 takes 200 threads per line: at most 1024 per block)
-    static constexpr int CB = sizeof(T) == 4 && M > 512 && 8 * PL::TPL <= 1024 ? 8 : 4;
+    static constexpr int CB = sizeof(T) == 8 ? (M > 768 ? 4 : 2) : M > 512 && 8 * PL::TPL <= 1024 ? 8 : 4;
     static constexpr int TR = (LB * PL::TPL + 63) / 64 * 64, TC = (CB * PL::TPL + 63) / 64 * 64;
     static constexpr size_t lds_rows = ((size_t)M + 2 * (size_t)LB * MixRow<T, M>::PITCH) * sizeof(cplx<T>);
     static constexpr bool ONE = sizeof(T) == 8 || M > 512;
