@@ -638,7 +638,11 @@ int wait_flag(const unsigned* flag, unsigned v, hipStream_t st) {
 // 1.73 ms for a 256^2 field (profiled with the runtime's hipMemcpy2D).
 // A call takes a buffer and gives it back once the GPU is done with it, so any
 // number of host threads may hold one each; what is kept between calls is
-// bounded and freed with the library's last handle.
+// bounded and freed with the library's last handle.  No call takes more than
+// STAGE_MAX: larger transfers go through it piece after piece, because pinning
+// memory is dear (75 MB of ice for 64 domains of 384^2, pinned and freed with
+// every update: 32.4 ms; in pieces 7.1, from pageable memory 7.4).
+constexpr size_t STAGE_MAX = (size_t)16 << 20;
 struct Stage {
     char* h = nullptr;      // host address
     char* d = nullptr;      // the same memory as the device sees it
@@ -649,10 +653,11 @@ struct Stage {
 };
 class StagePool {
     static constexpr size_t UNIT = (size_t)4 << 20, KEEP = (size_t)64 << 20;
+    static_assert(STAGE_MAX % UNIT == 0 && STAGE_MAX <= KEEP, "every buffer can be kept");
     std::mutex mu_;
-    std::vector<Stage> free_;
+    std::deque<Stage> free_;   // oldest first
     size_t kept_ = 0;
-    long long users_ = 0;
+    long long users_ = 0, made_ = 0;
 
 public:
     int take(size_t bytes, Stage& out) {
@@ -667,6 +672,7 @@ public:
                 free_.erase(free_.begin() + best);
                 return 0;
             }
+            ++made_;
         }
         Stage s;
         s.bytes = (bytes + UNIT - 1) / UNIT * UNIT;
@@ -679,24 +685,35 @@ public:
         out = s;
         return 0;
     }
+    // (the buffers given back last are kept: those are the sizes in use)
     void give(const Stage& s) {
         if (!s.h) return;
+        std::vector<Stage> out;
         {
             std::lock_guard<std::mutex> lk(mu_);
-            if (kept_ + s.bytes <= KEEP && users_ > 0) {
+            if (users_ > 0) {
                 free_.push_back(s);
                 kept_ += s.bytes;
-                return;
+            } else {
+                out.push_back(s);
+            }
+            for (; kept_ > KEEP; free_.pop_front()) {
+                out.push_back(free_.front());
+                kept_ -= free_.front().bytes;
             }
         }
-        (void)hipHostFree(s.h);
+        for (const Stage& o : out) (void)hipHostFree(o.h);
+    }
+    long long made() {
+        std::lock_guard<std::mutex> lk(mu_);
+        return made_;
     }
     void add_user() {
         std::lock_guard<std::mutex> lk(mu_);
         ++users_;
     }
     void drop_user() {
-        std::vector<Stage> out;
+        std::deque<Stage> out;
         {
             std::lock_guard<std::mutex> lk(mu_);
             if (--users_ > 0) return;
@@ -720,6 +737,48 @@ struct StageLease {
         g_stages.give(s);
     }
 };
+
+// Host fields to the device through pinned memory, all on the library stream:
+// the bus copies one while the host copies the next one.  Beyond STAGE_MAX the
+// buffer is used in turn in four pieces, each filled again once its last copy
+// has ended.  The caller keeps the lease until its stream has been waited for.
+struct Upload {
+    double* dst;
+    const double* src;
+    size_t bytes;
+};
+int upload(const std::vector<Upload>& list, StageLease& st) {
+    size_t total = 0;
+    for (const Upload& u : list) total += align256(u.bytes);
+    if (!total) return 0;
+    int rc = st.take(std::min(total, STAGE_MAX));
+    if (rc) return rc;
+    const bool whole = total <= STAGE_MAX;
+    constexpr size_t PIECE = STAGE_MAX / 4;
+    unsigned seq[4] = {};
+    size_t at = 0, piece = 0;   // next free byte, pieces filled so far
+    for (const Upload& u : list)
+        for (size_t done = 0; done < u.bytes;) {
+            size_t len = u.bytes - done;
+            if (!whole) {
+                if (at == PIECE) {
+                    // full: number its copies and go on in the next one
+                    launch_flag(st.s.flag_d(), seq[piece++ % 4] = next_seq(), g_stream);
+                    HIPCHK(hipGetLastError());
+                    at = 0;
+                    if (piece >= 4) rc = wait_flag(st.s.flag_h(), seq[piece % 4], g_stream);
+                    if (rc) return rc;
+                }
+                len = std::min(len, PIECE - at);
+            }
+            const size_t off = at + piece % 4 * PIECE;
+            std::memcpy(st.s.h + off, (const char*)u.src + done, len);
+            HIPCHK(hipMemcpyAsync((char*)u.dst + done, st.s.h + off, len, hipMemcpyHostToDevice, g_stream));
+            done += len;
+            at += whole ? align256(len) : len;
+        }
+    return 0;
+}
 
 // Concurrent sub-batches of the attempt loop (at most three streams besides
 // the library stream, default priority).  One launch of an attempt kernel
@@ -1164,24 +1223,30 @@ int read_window(fi_isos* h, const void* src, int bit, int i0, int j0, int ni, in
     constexpr size_t CHUNK = (size_t)512 << 10;
     const int rows = (int)std::max<size_t>(1, CHUNK / (sizeof(T) * ni));
     const int nch = (nj + rows - 1) / rows;
+    // chunk c lies in slot c % slots: all of them in the buffer up to STAGE_MAX
+    const size_t slot = (size_t)rows * ni;
+    const int slots = std::min(nch, (int)(STAGE_MAX / (sizeof(T) * slot)));
     StageLease st;
-    int rc = st.take(sizeof(T) * ni * nj);
+    int rc = st.take(std::min(sizeof(T) * (size_t)ni * nj, sizeof(T) * slot * slots));
     if (rc) return rc;
     // (numbers rise from chunk to chunk; another thread's may lie between)
     std::vector<unsigned> seq(nch);
-    for (int c = 0; c < nch; ++c) {
+    auto queue = [&](int c) -> int {
         const int j = c * rows, nr = std::min(rows, nj - j);
-        launch_crop(src, bit, h->n, i0, j0 + j, ni, nr, st.s.d + sizeof(T) * (size_t)j * ni, g_stream);
+        launch_crop(src, bit, h->n, i0, j0 + j, ni, nr, st.s.d + sizeof(T) * slot * (c % slots), g_stream);
         launch_flag(st.s.flag_d(), seq[c] = next_seq(), g_stream);
         HIPCHK(hipGetLastError());
-    }
-    for (int c = 0; c < nch; ++c) {
+        return 0;
+    };
+    for (int c = 0; c < slots && !rc; ++c) rc = queue(c);
+    for (int c = 0; c < nch && !rc; ++c) {
         const int j = c * rows, nr = std::min(rows, nj - j);
         rc = wait_flag(st.s.flag_h(), seq[c], g_stream);
-        if (rc) return rc;
-        const size_t at = (size_t)j * ni;
-        put(at, (size_t)nr * ni, (const T*)st.s.h + at);
+        if (rc) break;
+        put((size_t)j * ni, (size_t)nr * ni, (const T*)st.s.h + slot * (c % slots));
+        if (c + slots < nch) rc = queue(c + slots);
     }
+    if (rc) return rc;
     st.idle = true;
     return 0;
 }
@@ -1739,25 +1804,21 @@ int fi_isos_init_state(fi_isos* h, const double* z_bed, const double* H_ice, dou
     return 0;
 }
 
-// The caller's ice in pinned memory, where the update's first kernel reads it.
-static int stage_ice(const fi_isos* h, const double* H_ice, StageLease& ice) {
-    const size_t bytes = sizeof(double) * h->nx_ice * h->ny_ice;
-    int rc = ice.take(bytes);
-    if (rc) return rc;
-    std::memcpy(ice.s.h, H_ice, bytes);
-    return 0;
-}
-
 int fi_isos_update(fi_isos* h, const double* H_ice, double time, fi_bsl* b) {
     if (!h || !H_ice || !b) return fail(FI_E_ARG, "NULL argument");
     if (!h->state_init) return fail(FI_E_STATE, "isos_update called before isos_init_state");
     int rc = bind_bsl(h, b);
     if (rc) return rc;
+    // the ice in pinned memory, where the update's first kernel reads it, or
+    // (1448^2 cells and more) in H_in by way of it
+    const size_t bytes = sizeof(double) * h->nx_ice * h->ny_ice;
+    const bool direct = bytes <= STAGE_MAX;
     StageLease ice;
-    rc = stage_ice(h, H_ice, ice);
+    rc = direct ? ice.take(bytes) : upload({{h->hm.H_in, H_ice, bytes}}, ice);
     if (rc) return rc;
+    if (direct) std::memcpy(ice.s.h, H_ice, bytes);
     std::vector<fi_isos*> hs{h};
-    rc = run_update(hs, h->d_mem, h->shape, h->sb, time, true, nullptr, 1, (const double*)ice.s.d);
+    rc = run_update(hs, h->d_mem, h->shape, h->sb, time, true, nullptr, 1, direct ? (const double*)ice.s.d : nullptr);
     ice.idle = rc == 0;   // (the update's last readback has been waited for)
     return rc;
 }
@@ -2111,30 +2172,17 @@ int fi_batch_update(fi_batch* b, const double* const* H_ice, double time, fi_bsl
     if (!b || !bsl) return fail(FI_E_ARG, "NULL argument");
     const int nmem = (int)b->mem.size();
     bool dirty = false;
-    size_t ice_bytes = 0;
+    std::vector<Upload> ices;
     for (int m = 0; m < nmem; ++m) {
         fi_isos* h = b->mem[m];
         if (!h->state_init) return fail(FI_E_STATE, "member %d: update before init_state", m);
         if (!bsl[m]) return fail(FI_E_ARG, "member %d: bsl is NULL", m);
         if (b->hm[m].bsl != bsl[m]->d) { b->hm[m].bsl = bsl[m]->d; dirty = true; }
-        if (H_ice && H_ice[m]) ice_bytes += align256(sizeof(double) * h->nx_ice * h->ny_ice);
+        if (H_ice && H_ice[m]) ices.push_back({h->hm.H_in, H_ice[m], sizeof(double) * h->nx_ice * h->ny_ice});
     }
-    // member after member through pinned memory: the bus copies one member's
-    // ice while the host copies the next one's
     StageLease ice;
-    if (ice_bytes) {
-        int rc = ice.take(ice_bytes);
-        if (rc) return rc;
-        size_t off = 0;
-        for (int m = 0; m < nmem; ++m) {
-            if (!H_ice[m]) continue;
-            const fi_isos* h = b->mem[m];
-            const size_t bytes = sizeof(double) * h->nx_ice * h->ny_ice;
-            std::memcpy(ice.s.h + off, H_ice[m], bytes);
-            HIPCHK(hipMemcpyAsync(h->hm.H_in, ice.s.h + off, bytes, hipMemcpyHostToDevice, g_stream));
-            off += align256(bytes);
-        }
-    }
+    int rc = upload(ices, ice);
+    if (rc) return rc;
     // groups of members sharing a bsl object, in batch order
     for (int m = 0; m < nmem; ++m) {
         int prev = -1, next = -1;
@@ -2150,7 +2198,7 @@ int fi_batch_update(fi_batch* b, const double* const* H_ice, double time, fi_bsl
         }
     }
     if (dirty) HIPCHK(hipMemcpy(b->d_mem, b->hm.data(), sizeof(Member) * nmem, hipMemcpyHostToDevice));
-    const int rc = run_update(b->mem, b->d_mem, b->shape, b->sb, time, true);
+    rc = run_update(b->mem, b->d_mem, b->shape, b->sb, time, true);
     ice.idle = rc == 0;
     return rc;
 }
@@ -2800,6 +2848,12 @@ int fi_prof_fused(void) { return prof_fused(); }
 int fi_prof_shape(int* out) {
     if (!out) return fail(FI_E_ARG, "NULL argument");
     prof_shape(out);
+    return 0;
+}
+
+int fi_prof_pinned(long long* buffers) {
+    if (!buffers) return fail(FI_E_ARG, "NULL argument");
+    *buffers = g_stages.made();
     return 0;
 }
 

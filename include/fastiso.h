@@ -314,6 +314,9 @@ int fi_prof_shape(int* out);
 /* kernel = 99 in fi_prof_select times every attempt kernel; this sums the
  * timed launches of one of them (0, 2, 3; -1: all timed launches) */
 int fi_prof_collect_kernel(int kernel, double* total_ms, long long* launches);
+/* Pinned staging buffers allocated since the library was loaded: constant from
+ * update to update once the sizes in use have been seen. */
+int fi_prof_pinned(long long* buffers);
 /* Achieved device-to-device copy bandwidth (bytes read + written per second /
  * 1e9) of `reps` copies of `mib` MiB on the library stream: the practical
  * ceiling beside the HBM peak. */
