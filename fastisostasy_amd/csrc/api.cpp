@@ -990,6 +990,26 @@ int first_round_margin() {
     return m;
 }
 
+// Attempts of a first round: the estimate from dt, or as many as one of the last
+// four updates of the same span took (0: none).  A load that changes from one
+// coupling step to the next cuts the step at the start of each update, and then
+// the past is the better guess (N = 64 disc under varying ice: 6 to 9 attempts
+// where the last dt promises one); after one update of many attempts it is not.
+// So: the count that would have cost least for those updates and the estimate
+// together, at 25 us for a second round and 4 us for an unused attempt.
+int first_round(double need, const double (&past)[4]) {
+    double best = std::max(1.0, need), least = 1e300;
+    auto cost = [&](double a) {
+        double c = 0.0;
+        for (double p : past)
+            if (p > 0.0) c += p > a ? 25.0 : 4.0 * (a - p);
+        return c + (need > a ? 25.0 : 4.0 * (a - need));
+    };
+    for (double a : {best, past[0], past[1], past[2], past[3]})
+        if (a >= 1.0 && cost(a) < least) { best = a; least = cost(a); }
+    return (int)std::min(256.0, best);
+}
+
 int job_begin(UpdateJob& j) {
     const int nmem = (int)j.hs.size();
     const fi_isos& h0 = *j.hs[0];
@@ -1033,23 +1053,16 @@ int job_begin(UpdateJob& j) {
     // round launches as many attempts as the slowest member needs at the dt it
     // ended its previous update with, plus a margin for rejections; after each
     // readback job_more corrects the estimate.
-    // A load that changes from one coupling step to the next cuts the step at
-    // the start of each update: then the most attempts among the last four
-    // updates of the same span are the better guess (N = 64 disc under varying
-    // ice: 6 to 9 attempts where the last dt promises one).  Four, because a
-    // second round costs about 25 us and an unused attempt 4: with the last
-    // update plus one instead, every other update took a second round.
-    double need = 0.0, again = 0.0;
+    double need = 0.0, past[4] = {};
     for (int m = 0; m < nmem; ++m) {
         const fi_isos& h = *j.hs[m];
         const double span = j.t_of(m) - h.last_t;
         if (h.last_dt > 0.0) need = std::max(need, std::ceil(span / h.last_dt));
-        for (const auto& p : h.past)
-            if (std::fabs(span - p.span) <= 1e-6 * span) again = std::max(again, (double)p.attempts);
+        for (int k = 0; k < 4; ++k)
+            if (std::fabs(span - h.past[k].span) <= 1e-6 * span) past[k] = std::max(past[k], (double)h.past[k].attempts);
     }
     if (need > 0.0) need += (double)first_round_margin();
-    need = std::max(need, again);
-    j.ahead = (int)std::min(256.0, std::max(1.0, need));
+    j.ahead = first_round(need, past);
     // concurrent sub-batches only on the library stream (their streams are shared)
     j.K = shape.method == 3 && j.st == g_stream && j.subbatch ? sub_count(n, h0.fp64, nmem, j.ahead) : 1;
     if (j.K > 1) {
