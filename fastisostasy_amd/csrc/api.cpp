@@ -521,6 +521,7 @@ struct fi_isos {
     struct Past { double span = 0; long long attempts = 0; };
     Past past[4];                // years (0: unknown) and attempts of the last updates, newest first
     long long attempts_seen = 0;
+    bool dt_is_init = false;     // last_dt is dt_init: no update has been made
     int last_status = 0;         // status of the last update's instability and NaN checks
     char* arena = nullptr;
     size_t arena_bytes = 0;      // HBM footprint of the domain (one allocation)
@@ -1057,7 +1058,8 @@ int job_begin(UpdateJob& j) {
     for (int m = 0; m < nmem; ++m) {
         const fi_isos& h = *j.hs[m];
         const double span = j.t_of(m) - h.last_t;
-        if (h.last_dt > 0.0) need = std::max(need, std::ceil(span / h.last_dt));
+        // (dt_init promises little: beyond eight attempts a second round is cheaper)
+        if (h.last_dt > 0.0) need = std::max(need, std::min(std::ceil(span / h.last_dt), h.dt_is_init ? 8.0 : 256.0));
         for (int k = 0; k < 4; ++k)
             if (std::fabs(span - h.past[k].span) <= 1e-6 * span) past[k] = std::max(past[k], (double)h.past[k].attempts);
     }
@@ -1174,6 +1176,7 @@ int job_end(UpdateJob& j) {
         h->attempts_seen = c.attempts;
         h->last_t = c.t;
         h->last_dt = j.stepping ? c.dt : 0.0;
+        h->dt_is_init = false;
         const char* what;
         h->last_status = instability_status(c, what);
         if (h->last_status && !first) {
@@ -1811,6 +1814,7 @@ int fi_isos_init_state(fi_isos* h, const double* z_bed, const double* H_ice, dou
     // (the first update's launch estimate starts from dt_init)
     h->last_t = time;
     h->last_dt = h->par.dt_init;
+    h->dt_is_init = true;
     for (auto& p : h->past) p = {};
     h->state_init = true;
     h->use_restart = false;

@@ -1,6 +1,6 @@
 """How many attempts the host launches ahead of an update (more than it needs are
 idle launches of about 4 us each, fewer cost a second round of about 25 us):
-after a jump of the load."""
+after a jump of the load, and with a first step far too small."""
 import ctypes
 
 import numpy as np
@@ -55,3 +55,15 @@ def test_one_expensive_update_does_not_set_the_next_ones(monkeypatch):
     # at most what one saved and one unneeded round cost per update
     wasted = sum(4.0 * (launched - needed) + 25.0 * (rounds - 1) for launched, needed, rounds in after)
     assert wasted <= 50.0 * len(after), after
+
+
+@pytest.mark.parametrize("dt_init", [1e-3, 1.0])
+def test_first_step_far_too_small(dt_init):
+    nx, dx = 128, 25e3
+    h = G.IsosClass(G.make_params(**W.params(min_pad=1600e3, dt_init=dt_init)), nx, nx, dx)
+    b = G.bsl_init("const", 0.0)
+    h.init_state(np.full((nx, nx), 1e6), np.zeros((nx, nx)), 0.0, b)
+    launched, needed, rounds = _update(h, W.disc_load(nx, dx), 10.0, b)
+    print(f"dt_init {dt_init}: launched {launched}, needed {needed}, rounds {rounds}", flush=True)
+    # the first round takes at most eight and one for a rejection, later ones follow the step as it is
+    assert needed <= launched <= 2 * needed + 9
