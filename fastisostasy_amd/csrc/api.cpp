@@ -2190,16 +2190,18 @@ int fi_batch_update(fi_batch* b, const double* const* H_ice, double time, fi_bsl
     const int nmem = (int)b->mem.size();
     bool dirty = false;
     std::vector<Upload> ices;
+    // (every check before the first change: a refused call leaves the batch as it was)
     for (int m = 0; m < nmem; ++m) {
-        fi_isos* h = b->mem[m];
+        const fi_isos* h = b->mem[m];
         if (!h->state_init) return fail(FI_E_STATE, "member %d: update before init_state", m);
         if (!bsl[m]) return fail(FI_E_ARG, "member %d: bsl is NULL", m);
-        if (b->hm[m].bsl != bsl[m]->d) { b->hm[m].bsl = bsl[m]->d; dirty = true; }
         if (H_ice && H_ice[m]) ices.push_back({h->hm.H_in, H_ice[m], sizeof(double) * h->nx_ice * h->ny_ice});
     }
     StageLease ice;
     int rc = upload(ices, ice);
     if (rc) return rc;
+    for (int m = 0; m < nmem; ++m)
+        if (b->hm[m].bsl != bsl[m]->d) { b->hm[m].bsl = bsl[m]->d; dirty = true; }
     // groups of members sharing a bsl object, in batch order
     for (int m = 0; m < nmem; ++m) {
         int prev = -1, next = -1;
