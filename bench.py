@@ -34,12 +34,18 @@ FUSED_NAME = "kf_srow_fwd (stencil + forward row pass)"
 PROF_ALL = 99
 
 
-def fast_kernel_names(shape):
+def fast_kernel_names(shape, path=(0, 0, 0, -1)):
     """Template names (as rocprofv3 prints them) of the register-FFT attempt
     kernels the last timed attempt ran, from fi_prof_shape: {N, fp64, fused,
     fast, threads_row, C, row_tiles, srow_rows, threads_inv, dt_method,
-    column-pass exchange buffers}."""
+    column-pass exchange buffers}, and fi_prof_path: {two-launch attempts, their
+    line pairs per row block, per column block, convolution kernels}."""
     n, fp64, fused, fast, th, c, rt, rows, inv, meth, nbuf = shape
+    if path[0]:
+        # (kernel 0 is kt_turn too, in the launch that begins a round)
+        t = "double" if fp64 else "float"
+        turn = f"kt_turn<{t}, {n}, {path[1]}, true>"
+        return {0: turn, 2: f"kt_col<{t}, {n}, {path[2]}>", 3: turn}
     if not (fast and fused):
         return {}
     t = "double" if fp64 else "float"
@@ -53,8 +59,8 @@ def fast_kernel_names(shape):
 # Algorithmic HBM bytes per cell of the once-per-coupling-step kernels of an
 # LV-ELVA update without convolutions (uniform spacing, elastic and sea-surface
 # convolutions off: the ensemble workload), all FP64 but the FP32 copy of
-# canom_full and the 1-byte mask.  The per-domain scalar kernels (begin, bsl,
-# decide, corner, check, gather) move a few hundred bytes per domain.  The
+# canom_full and the 1-byte mask.  The per-domain scalar kernels (k_pre_bsl,
+# k_round_end, k_fin_check) move a few hundred bytes per domain.  The
 # FETCH_SIZE / WRITE_SIZE counters of the 64-member ensemble read 40.2 + 16.0,
 # 65.1 + 45.0 and 40.1 + 24.1 B/cell for these three.
 STEP_BYTES_PER_CELL = {
@@ -66,10 +72,10 @@ STEP_BYTES_PER_CELL = {
 }
 
 
-def step_roofline(cells, attempts_per_step, ms_per_step, s=4, peak=8000.0):
+def step_roofline(cells, attempts_per_step, ms_per_step, s=4, peak=8000.0, turn=False):
     """The coupling step as run (concurrent sub-batches, bookkeeping kernels
     included): algorithmic bytes of every kernel of a step over its wall time."""
-    attempt_b = sum(kernel_bytes_per_cell(k, s, True) for k in (0, 2, 3))
+    attempt_b = sum(kernel_bytes_per_cell(k, s, True, turn) for k in attempt_kernels(turn))
     per_cell = sum(STEP_BYTES_PER_CELL.values()) + attempt_b * attempts_per_step
     b = cells * per_cell
     gbs = b / (ms_per_step * 1e-3) / 1e9
@@ -94,11 +100,21 @@ def measured_traffic(kernel_name, cells):
     return k["read_bytes"] + k["write_bytes"]
 
 
-def kernel_bytes_per_cell(kernel, s, fused):
+def attempt_kernels(turn):
+    """Kernels launched once per attempt (two-launch attempts: kernel 0 only
+    begins a launch round)."""
+    return (2, 3) if turn else (0, 2, 3)
+
+
+def kernel_bytes_per_cell(kernel, s, fused, turn=False):
     """Algorithmic HBM bytes per cell per launch (s = bytes per RHS real).
 
     dwdt is written only by the attempt that reaches the coupling time, so the
     inverse row pass is priced without it."""
+    if turn and kernel == 3:
+        # kt_turn: read column pass's result, x (f64), D, 1/(2 eta), canom_full;
+        # write x2 (f64), row-transformed
+        return s + 8 + 3 * s + 8 + s
     if kernel == 0 and fused:
         return 8 + 3 * s + s       # read x (f64), D, 1/(2 eta), canom_full; write row-transformed
     return {0: 8 + 4 * s,          # read x (f64), D, 1/(2 eta), canom_full; write f
@@ -194,7 +210,10 @@ def run_batched(nmem, steps, warmup, precision, prof_kernel=None, timed=True, ex
         prof["fused"] = bool(load().fi_prof_fused())
         shape = (ctypes.c_int * 11)()
         check(load().fi_prof_shape(shape))
-        prof["names"] = fast_kernel_names(list(shape))
+        path = (ctypes.c_int * 4)()
+        check(load().fi_prof_path(path))
+        prof["turn"] = bool(path[0])
+        prof["names"] = fast_kernel_names(list(shape), list(path))
         check(load().fi_prof_select(-1))
     for _ in range(extra_steps):
         # untimed steps that bring a run to the end time of another
@@ -469,10 +488,11 @@ def kernel_roofline(prof, k, cells, n, fused):
     if cnt <= 0:
         return None
     avg_s = ms / cnt * 1e-3
-    nbytes = kernel_bytes_per_cell(k, 4, fused) * cells
+    turn = prof.get("turn", False)
+    nbytes = kernel_bytes_per_cell(k, 4, fused, turn) * cells
     achieved = nbytes / avg_s / 1e9
     full = prof.get("names", {}).get(k)
-    name = (FUSED_NAME if k == 0 else full.split("<")[0]) if (fused and full) else KERNEL_NAMES[k]
+    name = (FUSED_NAME if k == 0 and not turn else full.split("<")[0]) if (fused and full) else KERNEL_NAMES[k]
     traffic = measured_traffic(full, cells) if full else None
     return {"kernel": name, "template": full, "bytes_per_launch": nbytes, "avg_launch_us": round(avg_s * 1e6, 2), "launches": cnt,
             "achieved": round(achieved, 1), "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic}
@@ -480,18 +500,19 @@ def kernel_roofline(prof, k, cells, n, fused):
 
 def roofline(res, args, cells, n):
     """Roofline object: the dominant kernel (the fused stencil + forward row
-    pass) at the top level, every attempt kernel in `kernels`, and the three
-    transform passes together in `fft_passes` (their bytes over the sum of
-    their average launch times)."""
+    pass; kt_turn of two-launch attempts) at the top level, every attempt kernel
+    in `kernels`, and the transform passes together in `fft_passes` (their bytes
+    over the sum of their average launch times)."""
     prof = res["prof"]
     if not prof:
         return None
     fused = prof["fused"]
-    ks = {k: kernel_roofline(prof, k, cells, n, fused) for k in (0, 2, 3) if k in prof}
+    turn = prof.get("turn", False)
+    ks = {k: kernel_roofline(prof, k, cells, n, fused) for k in attempt_kernels(turn) if k in prof}
     ks = {k: v for k, v in ks.items() if v}
     if not ks:
         return None
-    top = ks.get(0) or next(iter(ks.values()))
+    top = ks.get(3 if turn else 0) or next(iter(ks.values()))
     out = {"kernel": top["kernel"], "template": top["template"], "bound": "hbm", "achieved": top["achieved"], "peak": HBM_PEAK_GBS,
            "unit": "GB/s", "frac": top["frac"], "traffic": top["traffic"], "avg_launch_us": top["avg_launch_us"],
            "launches": top["launches"], "bytes_per_launch": top["bytes_per_launch"]}
@@ -596,7 +617,7 @@ def main():
 
     roof = roofline(res, args, cells, n)
     roof["step"] = step_roofline(cells, res["attempts"] / args.members / (args.steps + args.warmup),
-                                 1e3 * res["wall"] / args.steps)
+                                 1e3 * res["wall"] / args.steps, turn=res["prof"]["turn"])
     single = {"workload": "one 256^2 ensemble member (N=256), 10-yr isos_update",
               "fp64": run_single("fp64", tune=not args.no_autotune),
               "mixed": run_single("mixed", tune=not args.no_autotune)}

@@ -2870,6 +2870,12 @@ int fi_prof_shape(int* out) {
     return 0;
 }
 
+int fi_prof_path(int* out) {
+    if (!out) return fail(FI_E_ARG, "NULL argument");
+    prof_path(out);
+    return 0;
+}
+
 int fi_prof_pinned(long long* buffers) {
     if (!buffers) return fail(FI_E_ARG, "NULL argument");
     *buffers = g_stages.made();

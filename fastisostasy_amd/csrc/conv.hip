@@ -199,7 +199,9 @@ ConvFn conv_find(int n, bool fp64) {
 
 template <typename T>
 static void conv_t(const Member* d_mem, int nmem, const ConvShape& s, int which, hipStream_t st) {
-    if (s.mix && s.mix(d_mem, nmem, s.tw, which, s.pair, st)) return;
+    const bool grouped = s.mix && s.mix(d_mem, nmem, s.tw, which, s.pair, st);
+    prof_conv(grouped ? 1 : 0);
+    if (grouped) return;
     const int n = s.n, H = n + 1;
     rows_r2c<T>(d_mem, nmem, s, which, st);
     hipLaunchKernelGGL(c_cols<T>, dim3((H + s.Cc - 1) / s.Cc, nmem), dim3(s.threads_col), lbytes<T>(s.m, s.Cc + 1), st,

@@ -85,6 +85,12 @@ int prof_collect_kernel(int kernel, double* total_ms, long long* launches);
 int set_error(int code, const char* msg);
 int prof_fused();
 void prof_shape(int* out);   // 11 ints, fi_prof_shape
+void prof_path(int* out);    // 4 ints, fi_prof_path
+// what a launcher notes there while launches are being timed: line pairs per
+// block of kt_turn / kt_col (0: the other attempt kernels; -1: as it is), and
+// the kernels of the last convolution (1 grouped register FFT, 0 LDS)
+void prof_turn(int LO, int C);
+void prof_conv(int grouped);
 bool prof_active();
 // a start/stop event pair when launches of `kernel` are being timed
 bool prof_pair(int kernel, hipEvent_t* start, hipEvent_t* stop);

@@ -494,6 +494,8 @@ struct Prof {
     size_t used = 0;
     std::atomic<bool> fused{false};   // last attempt ran the fused stencil + row kernel
     RhsShape last{};              // launch shape of the last attempt
+    int turn_LO = 0, turn_C = 0;  // its blocks of two-launch attempts (0: none)
+    int conv = -1;                // kernels of the last convolution (-1: none yet)
 };
 Prof g_prof;
 
@@ -516,6 +518,7 @@ bool prof_pair(int kernel, hipEvent_t* start, hipEvent_t* stop) {
 void prof_select(int kernel) {
     g_prof.kernel = kernel;
     g_prof.used = 0;
+    if (kernel >= 0) { g_prof.turn_LO = g_prof.turn_C = 0; g_prof.conv = -1; }
 }
 
 int prof_fused() { return g_prof.fused.load(std::memory_order_relaxed) ? 1 : 0; }
@@ -525,7 +528,21 @@ void prof_shape(int* out) {
                        s.row_tiles, s.srow_rows, s.threads_inv, s.dt_method, s.fast ? col_buffers(s) : 1};
     for (int i = 0; i < 11; ++i) out[i] = v[i];
 }
+void prof_path(int* out) {
+    out[0] = g_prof.turn_C > 0 ? 1 : 0;
+    out[1] = g_prof.turn_LO;
+    out[2] = g_prof.turn_C;
+    out[3] = g_prof.conv;
+}
 bool prof_active() { return g_prof.kernel >= 0; }
+void prof_turn(int LO, int C) {
+    if (!prof_active()) return;
+    if (LO >= 0) g_prof.turn_LO = LO;
+    if (C >= 0) g_prof.turn_C = C;
+}
+void prof_conv(int grouped) {
+    if (prof_active()) g_prof.conv = grouped;
+}
 
 int prof_collect_kernel(int kernel, double* total_ms, long long* launches) {
     double tot = 0.0;
@@ -579,6 +596,7 @@ void launch_attempt_t(const Member* d_mem, int nmem, const RhsShape& s, hipStrea
     const bool fused = s.fused && s.fast && s.uniform && launch_fast_pass(d_mem, nmem, s, st, 0);
     g_prof.fused.store(fused, std::memory_order_relaxed);
     if (g_prof.kernel >= 0) g_prof.last = s;   // profiling runs (one host thread): the timed launches' shape
+    prof_turn(0, 0);
     if (!fused) {
         if (s.uniform) launch_k(0, k_stencil_u<T>, gs, dim3(256), 0, st, d_mem);
         else launch_k(0, k_stencil<T, false>, gs, dim3(256), 0, st, d_mem);

@@ -668,6 +668,7 @@ bool turn_rows(const Member* d, int nmem, const RhsShape& s, hipStream_t st, int
     const bool first = which == 0;
     launch_k(first ? 0 : 3, kt_turn<T, N, LO, UNI>, dim3(TN::NB, nmem), dim3(TN::THREADS), TN::lds, st, d, s.tw,
              first ? 1 : 0, nmem, s.solo ? 1 : 0);
+    prof_turn(LO, -1);
     return true;
 }
 template <typename T, int N, int C>
@@ -677,6 +678,7 @@ bool turn_cols(const Member* d, int nmem, const RhsShape& s, hipStream_t st, int
     if (!ok || which < 0) return ok;
     launch_k(2, kt_col<T, N, C>, dim3(TC::NB + 1, nmem), dim3(TC::THREADS), TC::lds, st, d, s.tw, s.tw64, nmem,
              s.solo ? 1 : 0);
+    prof_turn(-1, C);
     return true;
 }
 

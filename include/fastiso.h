@@ -314,6 +314,12 @@ int fi_prof_shape(int* out);
 /* kernel = 99 in fi_prof_select times every attempt kernel; this sums the
  * timed launches of one of them (0, 2, 3; -1: all timed launches) */
 int fi_prof_collect_kernel(int kernel, double* total_ms, long long* launches);
+/* Kernels of the last attempt and convolution since fi_prof_select(kernel >= 0)
+ * (4 ints): {two-launch attempts, their line pairs per row block and per column
+ * block (0: other kernels), convolution on the grouped register FFT (0: LDS
+ * kernels, -1: none)}.  Under two-launch attempts kernel 0 is the forward part
+ * that begins a launch round, 2 the column pass, 3 the rest of the attempt. */
+int fi_prof_path(int* out);
 /* Pinned staging buffers allocated since the library was loaded: constant from
  * update to update once the sizes in use have been seen. */
 int fi_prof_pinned(long long* buffers);
