@@ -235,7 +235,7 @@ int make_three_pass_shape(int n, int nmem, bool fp64, bool uniform, bool tuned, 
         // the largest blocks that still give every CU one; no block below a
         // wave when a wave-sized one exists (one 256^2 domain: 2 line pairs);
         // FP64 at 4 line pairs, whose LDS lets four blocks share a CU (16 of
-        // 384^2: 75.3 us per attempt against 81.0 with 8)
+        // 384^2 in one launch: 72.2 us per attempt against 77.5 with 8)
         for (int C : {16, 8, 4, 2, 1}) {
             if (!col_ok(C) || (fp64 && C > 4)) continue;
             if (best_c && C * tpl < 64) break;
@@ -393,17 +393,27 @@ int make_three_pass_shape(int n, int nmem, bool fp64, bool uniform, bool tuned, 
 
 // Two-launch attempts (rhs_turn.hpp) for this group?  At the general lengths
 // always: they replace five launches of the mixed-radix LDS kernels (one
-// N = 320 domain, mixed: 15.6 us per attempt against 59.5; 64 of 200^2: 51.6
-// against 155).  At the lengths of the three-launch register kernels (2^k,
-// 3 * 2^k) while launches and not bytes set the pace, measured per attempt
-// (two launches against three, mixed): one 256^2 domain 13.3 / 16.9 us, 512^2
-// 16.5 / 19.8; 48 of 128^2 21.9 / 21.9, 12 of 256^2 23.6 / 23.5, 13 27.4 / 24.6
-// (FP64: 8 20.8 / 22.5, 10 31.3 / 29.9); 28 of 192^2 31.2 / 41.8 and 32 46.3 /
-// 45.7 (FP64: 28 40.1 / 52.3); 13 of 384^2 47.2 / 50.3 and 14 51.3 / 51.0
-// (FP64: 8 48.8 / 50.3, 16 90.6 / 81.0); 2 of 512^2 20.1 / 21.4 but 3 30.7 /
-// 27.6 and 2 in FP64 27.7 / 26.5.  A launch shape asked of the other kernels
-// (environment, autotuner) keeps those; FI_TURN = 0 never, 2 wherever the
-// kernels exist (tests).
+// N = 320 domain, mixed: 15.1 us per attempt against 58.3; 64 of 200^2: 49.8
+// against 124).  At the lengths of the three-launch register kernels (2^k,
+// 3 * 2^k) while launches and not bytes set the pace, in us per attempt (two
+// launches / three):
+//            mixed                                FP64
+//    64^2    192 18.8 / 22.0, 384 29.8 / 31       128 18.6 / 24, 256 29.0 / 30.5
+//   128^2    31 17.9 / 18.8, 96 29.2 / 29-32      31 21.6 / 22.2, 64 31.5 / 30.2
+//   256^2    1 12.8 / 15.8, 12 20.6 / 21.8,       1 14.4 / 17.7, 8 19.4 / 21.1,
+//            13 24.3 / 22.8                       9 27.6 / 26.9
+//   512^2    1 16.6 / 19.4, 2 18.0 / 20.1,        1 20.5 / 23.0, 2 24.7 / 25.4
+//            3 26.0 / 25.1
+//   192^2    28 29.8 / 41.9                       28 42.4 / 51.9
+//   384^2    1 15.1 / 22.9, 13 42.9 / 48.0,       4 31.3 / 37.2, 8 45.4 / 47.4,
+//            14 46.6 / 48.7                       9 54.4 / 48.7
+// (from 32 domains as two sub-batches).  The 3 * 2^k lengths have limits of
+// their own because their three-launch kernels take up to twice as long per cell
+// (28 of 192^2 against 16 of 256^2), 512^2 because one block of its rows fills a
+// CU's LDS.  The limits at 192^2 (31 30.7 / 43.3), of mixed 384^2 and of FP64
+// 512^2 lie below the crossing.  A launch shape asked of the
+// other kernels (environment, autotuner) keeps those; FI_TURN = 0 never, 2
+// wherever the kernels exist (tests).
 //
 // Blocks: one line pair per kt_turn block while that leaves CUs idle otherwise
 // (two from 192 half-pairs of lines on, 160 in FP64: 2 of 512^2 20.1 us
@@ -412,14 +422,20 @@ int make_three_pass_shape(int n, int nmem, bool fp64, bool uniform, bool tuned, 
 // 16.6 us against 18.5 with eight), eight beyond (12 of 256^2 23.5 against
 // 25.8) and, up to N = 128, where two line pairs fill half a wave, from 192 on
 // (16 of 128^2 beside other groups: 1.4% of a serving mix of 40 domains).
-long long turn_cells(int n, bool fp64) {
+//
+// The limits are those of a launch alone.  Beside another sub-batch they hold
+// too (two of 24 of 128^2 in FP64 25.5 us against 27.2, two of 22 of 192^2 47.3 /
+// 59.3; two of 32 of 128^2 are the worst, 31.1 / 29.7), except where one block
+// fills a CU's LDS: FP64 at N = 384, two of 5 and 6 56.8 / 57.6, two of 6
+// 64.9 / 59.3, two of 8 77.3 / 61.0.
+long long turn_cells(int n, bool fp64, bool beside) {
     if (n == 192) return 28 * 192 * 192;
-    if (n == 384) return (fp64 ? 8 : 13) * 384 * 384;
+    if (n == 384) return (fp64 ? (beside ? 5 : 8) : 13) * 384 * 384;
     if (n == 512) return fp64 ? 1 << 18 : 1 << 19;
     return fp64 ? 8 << 16 : 12 << 16;
 }
 
-void turn_shape(int n, int nmem, bool fp64, bool uniform, bool tuned, const TunedShape& ts, RhsShape& s) {
+void turn_shape(int n, int nmem, bool fp64, bool uniform, bool beside, bool tuned, const TunedShape& ts, RhsShape& s) {
     s.turn = nullptr;
     s.turn_C = s.turn_LO = 2;
     for (const char* e : {"FI_GENERIC_FFT", "FI_GEN_LINES", "FI_NO_FUSED_STENCIL", "FI_SROW_ROWS", "FI_INV_THREADS",
@@ -430,7 +446,7 @@ void turn_shape(int n, int nmem, bool fp64, bool uniform, bool tuned, const Tune
     if (want == 0) return;
     if (tuned && (ts.threads_row || ts.C || ts.row_tiles || ts.gL || ts.gC || ts.srow_rows || ts.threads_inv)) return;
     const long long blocks = (long long)(n / 4) * nmem;
-    if (s.fast && want != 2 && (long long)n * n * nmem > turn_cells(n, fp64)) return;
+    if (s.fast && want != 2 && (long long)n * n * nmem > turn_cells(n, fp64, beside)) return;
     s.turn_C = blocks > (n <= 128 ? 191 : 512) ? 8 : 2;
     s.turn_LO = blocks >= (fp64 ? 160 : 192) ? 2 : 1;
     // FI_TURN_LO = 1 | 2, FI_TURN_C = 2 | 8 override the blocks (tuning)
@@ -441,12 +457,13 @@ void turn_shape(int n, int nmem, bool fp64, bool uniform, bool tuned, const Tune
     if (f && f(nullptr, nmem, s, nullptr, -1)) s.turn = f;
 }
 
-// Row / column blocking for a batch of `nmem` domains of size n.
-int make_shape(int n, int nmem, bool fp64, bool uniform, RhsShape& s) {
+// Row / column blocking for a batch of `nmem` domains of size n (beside: other
+// sub-batches run at the same time).
+int make_shape(int n, int nmem, bool fp64, bool uniform, RhsShape& s, bool beside = false) {
     TunedShape ts;
     const bool tuned = tuned_for(n, fp64, nmem, ts);
     int rc = make_three_pass_shape(n, nmem, fp64, uniform, tuned, ts, s);
-    if (!rc) turn_shape(n, nmem, fp64, uniform, tuned, ts, s);
+    if (!rc) turn_shape(n, nmem, fp64, uniform, beside, tuned, ts, s);
     return rc;
 }
 
@@ -492,9 +509,9 @@ int make_conv_shape(int n, bool fp64, ConvShape& s) {
 
 }  // namespace
 
-// Summary buffer of a launch group: pinned, coherent host memory that the
-// gather kernel stores to directly through its device address `d`, so a
-// round's readback is that kernel alone (no blit copy queued behind it).
+// Summary buffer of a launch group: pinned, coherent host memory that the last
+// kernel of a round (k_fin_check) stores to directly through its device address
+// `d`, so the readback needs no copy queued behind it.
 struct SumBuf {
     CtlSummary* d = nullptr;
     CtlSummary* h = nullptr;
@@ -808,10 +825,11 @@ int ensure_sub(int k) {
 
 // number of sub-batches for a batch of nmem domains about to run `ahead`
 // attempts (the autotuner's choice, else 2 from 32 domains, and in FP64 off 2^k
-// from 1.5 million cells: 16 of 384^2 72.3 us per attempt against 81.0, 16 of 320^2
-// 69.5 against 78.7 -- while 8 of 512^2 lose, 56.7 against 50.6; FI_SUBBATCHES
-// overrides).  Splitting and joining the streams costs as much as a dozen
-// attempts gain.
+// from 1.5 million cells, us per attempt against one launch: 12 of 384^2 59.5 /
+// 69.0, 16 61.0 / 72.1, 16 of 320^2 67.1 / 75.1, 8 of 448^2 61.4 / 65.7, but
+// 10 of 384^2 52.3 / 50.2; at 2^k less, 8 of 512^2 49.5 / 52.1, 12 69.1 / 70.7;
+// FI_SUBBATCHES overrides).  Splitting and joining the streams costs as much as
+// a dozen attempts gain.
 int sub_count(int n, bool fp64, int nmem, int ahead) {
     const bool large = fp64 && (n & (n - 1)) != 0 && nmem >= 8 && (long long)n * n * nmem >= 3 << 19;
     int k = nmem >= 32 || (large && ahead >= 16) ? 2 : 1;
@@ -830,7 +848,7 @@ int sub_shape(int n, int nsub, bool fp64, bool uniform, int dt_method, const Rhs
         // a shape under trial is not cached
         RhsShape& s = t_trial_sub[k];
         s = RhsShape{};
-        int rc = make_shape(n, nsub, fp64, uniform, s);
+        int rc = make_shape(n, nsub, fp64, uniform, s, true);
         if (rc) return rc;
         s.dt_method = dt_method;
         out = &s;
@@ -842,7 +860,7 @@ int sub_shape(int n, int nsub, bool fp64, bool uniform, int dt_method, const Rhs
     if (it == g_sub_shapes.end()) {
         RhsShape s{};
         g_mu.unlock();
-        int rc = make_shape(n, nsub, fp64, uniform, s);
+        int rc = make_shape(n, nsub, fp64, uniform, s, true);
         g_mu.lock();
         if (rc) return rc;
         s.dt_method = dt_method;

@@ -126,6 +126,24 @@ def test_split_that_depends_on_the_attempts_ahead(monkeypatch):
         assert all(np.array_equal(x, y) for x, y in zip(f0, f1))
 
 
+def test_sub_batches_have_their_own_limit(monkeypatch):
+    """At FP64 384^2 one block of the two-launch attempts fills a CU's LDS: eight
+    domains take them alone, not beside another sub-batch of eight."""
+    def run(members):
+        doms = [make_domain(384, "fp64", False, m) for m in range(members)]
+        bat = G.Batch([d[0] for d in doms])
+        for t in (0.5, 8.5):   # (the second update launches more than sixteen attempts ahead)
+            bat.update(t, [d[1] for d in doms], [d[2] for d in doms])
+        bat.close()
+
+    print("case: 8 and 16 of 384^2 fp64", flush=True)
+    _clear(monkeypatch)
+    assert _profiled(lambda: run(8))[1][0] == 1
+    assert _profiled(lambda: run(16))[1][0] == 0
+    _clear(monkeypatch, FI_SUBBATCHES="2")
+    assert _profiled(lambda: run(10))[1][0] == 1
+
+
 @pytest.mark.parametrize("method", [1, 2])
 def test_relaxation_rounds_with_rejected_steps(method, monkeypatch):
     """One-launch relaxation attempts over more than one launch round per
