@@ -181,9 +181,10 @@ void small_batch_shape(RhsShape& s, int nmem, bool tuned, const TunedShape& ts, 
         // the row blocks hold fewer threads than columns: one column per thread
         // keeps the march's window in registers)
         // (8 rows while 16-row blocks would leave CUs idle, at 2^k while they
-        // would give each fewer than two: 4 of 512^2 24.6 us per attempt against
-        // 26.3 in 4-row blocks, 16 of 256^2 24.1 against 25.0 in 16-row ones; 12
-        // of 384^2 47.6 in 16-row blocks against 49.5)
+        // would give each fewer than two, us per attempt in blocks of 4 / 8 / 16
+        // rows: 4 of 512^2 24.9 / 23.3 / 26.1, 16 of 256^2 23.6 / 22.9 / 23.6; 14 of
+        // 384^2 54.9 / 50.3 / 48.6, 20 66.0 / 57.9 / 52.9: there the halo rows that
+        // smaller blocks repeat cost more than the fuller chip gives)
         int r = tuned && ts.srow_rows ? ts.srow_rows
                 : short_of(4, 256)    ? 2
                 : short_of(8, 256)    ? 4
@@ -416,12 +417,13 @@ int make_three_pass_shape(int n, int nmem, bool fp64, bool uniform, bool tuned, 
 // wherever the kernels exist (tests).
 //
 // Blocks: one line pair per kt_turn block while that leaves CUs idle otherwise
-// (two from 192 half-pairs of lines on, 160 in FP64: 2 of 512^2 20.1 us
-// against 21.4, 2 of 320^2 in FP64 19.6 against 20.6, but one 512^2 domain 16.9
-// against 18.1), two line pairs per kt_col block up to 512 of them (8 of 256^2
-// 16.6 us against 18.5 with eight), eight beyond (12 of 256^2 23.5 against
-// 25.8) and, up to N = 128, where two line pairs fill half a wave, from 192 on
-// (16 of 128^2 beside other groups: 1.4% of a serving mix of 40 domains).
+// (two from 192 half-pairs of lines on, 160 in FP64, us per attempt with one /
+// two: one 512^2 domain 16.6 / 17.7, two 19.2 / 17.9, one of 320^2 in FP64 17.9 /
+// 19.4, two 20.1 / 19.2); distorted grids always two, the only block their kernels
+// exist with.  Two line pairs per kt_col block up to 512 of them (8 of 256^2
+// 15.4 us against 17.2 with eight; 12 19.4 against 20.6 too: the line lies low),
+// eight beyond and, up to N = 128, where two line pairs fill half a wave, from 192 on
+// (16 of 128^2 14.2 both; beside other groups 1.4% of a serving mix of 40 domains).
 //
 // The limits are those of a launch alone.  Beside another sub-batch they hold
 // too (two of 24 of 128^2 in FP64 25.5 us against 27.2, two of 22 of 192^2 47.3 /
@@ -448,9 +450,9 @@ void turn_shape(int n, int nmem, bool fp64, bool uniform, bool beside, bool tune
     const long long blocks = (long long)(n / 4) * nmem;
     if (s.fast && want != 2 && (long long)n * n * nmem > turn_cells(n, fp64, beside)) return;
     s.turn_C = blocks > (n <= 128 ? 191 : 512) ? 8 : 2;
-    s.turn_LO = blocks >= (fp64 ? 160 : 192) ? 2 : 1;
+    s.turn_LO = !uniform || blocks >= (fp64 ? 160 : 192) ? 2 : 1;
     // FI_TURN_LO = 1 | 2, FI_TURN_C = 2 | 8 override the blocks (tuning)
-    if (const char* e = std::getenv("FI_TURN_LO")) s.turn_LO = std::atoi(e) == 1 ? 1 : 2;
+    if (const char* e = std::getenv("FI_TURN_LO")) s.turn_LO = std::atoi(e) == 1 && uniform ? 1 : 2;
     if (const char* e = std::getenv("FI_TURN_C")) s.turn_C = std::atoi(e) == 8 ? 8 : 2;
     TurnFn f = turn_find(n, fp64);
     // (a device that refuses the kernels' LDS keeps the others)
@@ -872,13 +874,14 @@ int sub_shape(int n, int nsub, bool fp64, bool uniform, int dt_method, const Rhs
 
 // Attempt graphs: a block of GRAPH_REPS attempted steps captured once per
 // (descriptor array, batch size, shape, stream) and replayed with one
-// hipGraphLaunch, so the host issues one call instead of 4 x GRAPH_REPS
-// kernel launches.  Kernel nodes only (no memset or copy nodes); the kernels
+// hipGraphLaunch, so the host issues one call instead of 16 to 32 kernel
+// launches.  Kernel nodes only (no memset or copy nodes); the kernels
 // read the descriptors and the control block at run time, so one graph
 // serves every update of a batch.  Opt-in for batches and single domains
-// (FI_GRAPHS=1): measured on the 64-member ensemble they are neutral (the
-// GPU, not the host, bounds the attempt rate) and rocprofv3's kernel tracing
-// crashed the host process inside a graph launch.  Benchmark kernel timing
+// (FI_GRAPHS=1): the GPU, not the host, bounds the attempt rate, and a replay
+// costs more than plain launches (us per attempt: one 256^2 domain 13.4 against
+// 12.8, 320^2 15.9 / 15.2, 16 of 256^2 23.8 / 23.1, 64 49.8 / 48.6); rocprofv3's
+// kernel tracing crashed the host process inside a graph launch.  Benchmark kernel timing
 // and round-based serving (whose groupings change every round) never use
 // them; polled serving does for groups of one or two domains, where the host's
 // launches would otherwise set the pace (FI_SERVER_GRAPHS=0 turns that off,
@@ -2772,11 +2775,13 @@ int fi_server_poll(fi_server* s, int wait, int* completed) {
             j.times = l.times.data();
             j.stepping = true;
             // Attempt graphs for groups of one or two domains: one host call per
-            // 8 attempts instead of 24 launches, so that enqueueing a group does
-            // not hold up the launch of the next (serving mix at 1.2x the
-            // unbatched capacity: p50 1.42 ms against 1.92); each lane stages in
-            // its own range, so a graph serves every later group of its size
-            // and shape on that lane.  FI_SERVER_GRAPHS=0 keeps plain launches.
+            // 8 attempts instead of 16 or 24 launches, so that enqueueing a group
+            // does not hold up the launch of the next (serving mix at 1.2x the
+            // unbatched capacity, two launches per attempt: p50 1.04 ms against
+            // 1.25, capacity 12.9 against 12.7 thousand requests/s; one 256^2 domain
+            // alone on the server 2.80 ms for four updates against 2.67); each lane
+            // stages in its own range, so a graph serves every later group of its
+            // size and shape on that lane.  FI_SERVER_GRAPHS=0 keeps plain launches.
             static const bool lane_graphs = [] {
                 const char* e = std::getenv("FI_SERVER_GRAPHS");
                 return !(e && std::atoi(e) == 0);

@@ -24,11 +24,12 @@ template <typename T, int M> struct ConvMix {
     static constexpr int N = M / 2, H = N + 1, C0 = N / 2 - 1;   // crop start (convolutions.f90:34-39), N even
     // rows: lines per block for about 256 threads;  columns: measured (us, one
     // domain / 16): FP64 M = 1024 with 4 columns and one exchange buffer 13.1 /
-    // 140 (two columns and two buffers: 21.9 / 216, one block per CU); a coupling
-    // step with two columns and one buffer: FP64 N = 153 192 us against 197, 240
-    // 194.5 / 196.5, 16 of 384^2 1440 / 1465, but N = 512 347 / 342; FP32 M = 1024
-    // with 8 columns and one buffer 9.3 / 74 (4 and two 9.6 / 110); short FP32
-    // lines with 4 and two buffers 6.2 / 19.3
+    // 140 (two columns and two buffers: 21.9 / 216, one block per CU); shorter
+    // FP64 lines with two columns against four, one buffer: M = 320 5.2 / 5.5 for
+    // one domain, 480 6.5 / 7.3, 600 8.5 / 9.5, 768 7.7 / 8.1, 16 of 480 22.5 / 26.0,
+    // of 768 39.0 / 47.9 (but 16 of 320 12.4 / 10.6, of 600 37 / 34, and 4 of 768
+    // 16.2 / 14.6); FP32 M = 1024 with 8 columns and one buffer 9.3 / 74 (4 and two
+    // 9.6 / 110); short FP32 lines with 4 and two buffers 6.2 / 19.3
     static constexpr int LB = PL::TPL >= 128 ? 2 : 256 / PL::TPL > 8 ? 8 : 256 / PL::TPL;
     // (M = 1000 takes 200 threads per line: at most 1024 per block)
     static constexpr int CB = sizeof(T) == 8 ? (M > 768 ? 4 : 2) : M > 512 && 8 * PL::TPL <= 1024 ? 8 : 4;

@@ -242,46 +242,6 @@ __device__ __forceinline__ void xcd_order(int per, int nmem, int& member, int& b
 }
 __device__ __forceinline__ void xcd_order(int& member, int& blk) { xcd_order(gridDim.x, gridDim.y, member, blk); }
 
-// Reduce the per-thread row statistics of two rows over the TPL threads of a
-// line with a fixed butterfly (lines wider than a wave combine their wave
-// halves through LDS in wave order; lines of 3 * 2^j threads combine their
-// three 2^j-lane groups through LDS in group order), and store them as the
-// row's partials.  The pattern depends on N alone, so the error norm of a
-// domain does not depend on how many domains share the launch.
-template <int TPL>
-__device__ __forceinline__ void row_reduce_store(double a1a, double a2a, double s2a, double a1b, double a2b,
-                                                 double s2b, int line, int t, gmut<double> pa,
-                                                 bool store = true) {
-    constexpr bool P2 = (TPL & (TPL - 1)) == 0;
-    constexpr int G = P2 ? TPL : TPL / 3;                  // lanes reduced by shuffles
-    static_assert(P2 || (G * 3 == TPL && (G & (G - 1)) == 0 && G <= 64), "TPL = 2^j or 3 * 2^j");
-    constexpr int W = G < 64 ? G : 64;
-    // (only the largest of the four maxima is used: one butterfly for them)
-    a1a = lanes_max<W>(fmax(fmax(a1a, a2a), fmax(a1b, a2b)));
-    s2a = lanes_sum<W>(s2a);
-    s2b = lanes_sum<W>(s2b);
-    constexpr int NG = P2 ? (TPL > 64 ? TPL / 64 : 1) : 3;   // groups combined through LDS
-    if constexpr (NG > 1) {
-        __shared__ double red[16][NG][3];
-        if ((t % W) == 0) {
-            double* r = red[line][t / W];
-            r[0] = a1a; r[1] = s2a; r[2] = s2b;
-        }
-        __syncthreads();
-        if (t == 0) {
-            for (int w = 1; w < NG; ++w) {
-                const double* r = red[line][w];
-                a1a = fmax(a1a, r[0]); s2a += r[1]; s2b += r[2];
-            }
-        }
-    }
-    if (t == 0 && store) {
-        // one entry per line: rows 2j and 2j+1 combined in a fixed order
-        pa[0] = a1a;
-        pa[1] = s2a + s2b;
-    }
-}
-
 // Stand-alone decision of one domain (one wave): applies the pending
 // decision of the last attempt, if any.
 __device__ __forceinline__ void decide_wave(const Member& M, int nblk) {

@@ -76,8 +76,7 @@ template <int N> __device__ __forceinline__ int turn_at(int row, int c) {
 // The arrays of a member: from the Member's own address for a single domain,
 // so that its first loads wait for no descriptor (with the kernel's arguments
 // preloaded into scalar registers: one 256^2 domain 13.8 -> 13.4 us per
-// attempt, 512^2 17.0 -> 16.5, N = 64 coupling step 153 -> 144 us), else from
-// the descriptor.
+// attempt, 512^2 17.0 -> 16.5), else from the descriptor.
 struct TurnPtrs {
     Ctl *ctl, *ctl_next;
     PhysDev* phys;
@@ -518,8 +517,8 @@ __global__ void __launch_bounds__((TurnCol<T, N, C>::THREADS)) kt_col(const Memb
     int mi, cblk;
     // -- but spread over all of them while there are fewer than nine blocks for
     // each: the few lines then come through eight L2 caches at once (one 512^2
-    // domain 16.5 -> 16.3 us per attempt in order, 6 of 300^2 30.7 -> 28.8, 2 of
-    // 512^2 23.1 -> 21.4; one 256^2 13.2 -> 13.3, N = 64 coupling step 104 -> 106)
+    // domain 16.5 -> 16.3 us per attempt in XCD order, 6 of 300^2 30.7 -> 28.8, 2 of
+    // 512^2 23.1 -> 21.4, but one 256^2 domain, 65 blocks, 13.2 -> 13.3)
     mi = blockIdx.y;
     cblk = blockIdx.x;
     if ((TurnCol<T, N, C>::NB + 1) * nmem >= 72) xcd_order(TurnCol<T, N, C>::NB + 1, nmem, mi, cblk);
